@@ -219,8 +219,9 @@ typedef struct ltx_linear_args {
     float *sumsq;
     int64_t sumsq_rs;
     /* Device scratch for the fp32 partial tiles of a split tail (see
-     * ltx_linear_workspace_bytes), 256-byte aligned, or NULL. With less than that the tail
-     * tiles run whole: same result up to fp32 summation order, slower. */
+     * ltx_linear_workspace_bytes), or for the statistic's column sums of a call too small to
+     * fill the CUs with 256 x 256 tiles, 256-byte aligned, or NULL. With less than that the
+     * 256 x 256 tiles run whole: same result up to fp32 summation order, slower. */
     void *workspace;
     size_t workspace_bytes;
     /* 0 = split the tail for the current device's CU count; n > 0 = for n resident workgroups

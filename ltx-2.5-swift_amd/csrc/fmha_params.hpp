@@ -128,6 +128,9 @@ struct LinearParams {
     int32_t grid;
 };
 
+// Tiles of linear_ks.hip, whose waves split the reduction: rows x columns of y.
+enum LinearKsTile { kLinearKs128 = 1, kLinearKs64 = 2, kLinearKs64x32 = 3, kLinearKs32 = 4 };
+
 // RMS statistic from partial sums of squares: rstd[row] = 1/sqrt(sum_j parts[row][j] / n + eps)
 // for rows [0, rows); parts row r at sumsq + r*rs, `blocks` partials.
 struct RstdParams {
@@ -216,6 +219,10 @@ int launch_combine(const CombineParams &p, int D, void *stream);
 int launch_passthrough(const PassParams &p, int D, void *stream);
 int launch_rstd(const RstdParams &p, void *stream);
 int launch_linear(const LinearParams &p, void *stream);           // linear_gemm.hip
+// linear_ks.hip: every tile whole, in tiles of LinearKsTile; p.part (float [M][column tiles])
+// when p.sumsq is set and the call has more than one column tile. p.tiles_*, n_full, splits
+// and grid are not read.
+int launch_linear_ks(const LinearParams &p, int tile, void *stream);
 int64_t linear_part_bytes(int64_t tail_tiles, int splits);          // one range: 256 KiB
 int launch_gemma_prep(const GemmaPrepParams &p, int D, void *stream);   // gemma_attn.hip
 int launch_gemma_attn(const GemmaAttnParams &p, int D, void *stream);

@@ -786,6 +786,7 @@ namespace {
 // written and read back by the fixup, about 0.116 us at 4.5 TB/s). Measured at 12480 x 4096 x
 // 4096 (16 tail tiles): 8 ranges 0.373 ms, 16 ranges (every CU busy) 0.382 ms. Pure host
 // arithmetic.
+constexpr double kLinearStepUs = 1.3, kLinearPartUs = 0.116;
 struct LinearSplit {
     int64_t tiles = 0, n_full = 0;
     int32_t splits = 1, steps_per_split = 0;
@@ -803,13 +804,12 @@ LinearSplit linear_split(int64_t M, int64_t N, int64_t K,
     const int64_t rem = T % groups;
     if (T == 0 || rem == 0 || 2 * rem > groups || nsteps < 4) return ls;
     const int64_t s_max = std::min<int64_t>(groups / rem, nsteps / 2);
-    constexpr double kStepUs = 1.3, kPartUs = 0.116;
     int64_t s = 1, per = nsteps;
     double best = 0.0;
     for (int64_t c = 2; c <= s_max; ++c) {
         const int64_t cp = (nsteps + c - 1) / c;
         const int64_t cs = (nsteps + cp - 1) / cp;   // no empty range
-        const double t = (double)cp * kStepUs + (double)(rem * cs) * kPartUs;
+        const double t = (double)cp * kLinearStepUs + (double)(rem * cs) * kLinearPartUs;
         if (s == 1 || t < best - 1e-9) {
             best = t;
             s = cs;
@@ -822,6 +822,34 @@ LinearSplit linear_split(int64_t M, int64_t N, int64_t K,
     ls.steps_per_split = (int32_t)per;
     ls.bytes = (size_t)ltx::linear_part_bytes(rem, (int)s);
     return ls;
+}
+
+// Tile of linear_ks.hip for a call none of whose 256 x 256 tiles runs whole (`ls`), or 0: the
+// k ranges and their fixup stay the cheaper. Both sides are estimated in us: the ranges as
+// linear_split does, plus 13 for their two launches; a ks tile by its rounds over the CUs, each
+// K / 64 steps at the tile's rate (measured over M 13 .. 3120, N 32 .. 12288, K 2048 and
+// 4096; a round takes longer the larger the tile, but feeds more products per byte staged), and
+// reading x and w once. Measured, ranges -> ks: 126 x 2048 x 2048 31 -> 9 us (32 x 32),
+// 12480 x 32 x 4096 52 -> 22.6 (64 x 32), 200 x 4096 x 4096 38 -> 15 (64 x 64),
+// 1024 x 4096 x 4096 61 -> 36 and 2048 x 4096 x 4096 89 -> 70 (128 x 128); 512 x 12288 x 4096
+// stays with the ranges (77.5 against 82.6).
+int linear_ks_tile(int64_t M, int64_t N, int64_t K, int64_t groups, const LinearSplit &ls) {
+    const double steps = (double)(K / 64), stream = 8.0 + 2e-6 * (double)((M + N) * K) / 5.0;
+    double best = 13.0 + ls.steps_per_split * kLinearStepUs +
+                  (double)(ls.tiles * ls.splits) * kLinearPartUs;
+    int tile = 0;
+    const struct { int tile; int64_t rows, cols; double step_us; } kTiles[] = {
+        {ltx::kLinearKs128, 128, 128, 0.38}, {ltx::kLinearKs64, 64, 64, 0.23},
+        {ltx::kLinearKs64x32, 64, 32, 0.16}, {ltx::kLinearKs32, 32, 32, 0.10}};
+    for (const auto &t : kTiles) {
+        const int64_t n = ((M + t.rows - 1) / t.rows) * ((N + t.cols - 1) / t.cols);
+        const double us = stream + (double)((n + groups - 1) / groups) * steps * t.step_us;
+        if (us < best) {
+            best = us;
+            tile = t.tile;
+        }
+    }
+    return tile;
 }
 
 }  // namespace
@@ -910,6 +938,14 @@ ltx_attn_status ltx_linear(const ltx_linear_args *a, void *stream) {
             (a->sumsq && overlaps(span(a->sumsq, a->M, a->sumsq_rs, blocks, 4))))
             return fail(LTX_ATTN_EINVAL, "linear workspace overlaps x, w, y or sumsq");
         p.part = (float *)a->workspace;
+        // (the statistic's column sums take far less of the workspace than the ranges would)
+        if (ls.n_full == 0)
+            if (const int tile = linear_ks_tile(a->M, a->N, a->K, groups, ls)) {
+                if (int e = ltx::launch_linear_ks(p, tile, stream))
+                    return fail(LTX_ATTN_EHIP, "linear launch: %s",
+                                hipGetErrorString((hipError_t)e));
+                return LTX_ATTN_OK;
+            }
         p.n_full = (int32_t)ls.n_full;
         p.splits = ls.splits;
         p.steps_per_split = ls.steps_per_split;

@@ -307,6 +307,39 @@ def test_persistent_grid_walks_many_tiles(device, K, groups):
     check_partials(p_few.cpu().numpy(), yb, f"K {K} on {groups} groups")
 
 
+@pytest.mark.parametrize("M,N,K,groups,bias", [
+    (33, 40, 320, 0, True),       # 32 x 32 tiles, ragged both ways; an odd number of k steps
+    (13, 2048, 2048, 0, True),    # one row tile, the statistic over 8 column tiles a block
+    (100, 1600, 320, 100, True),  # 64 x 32 tiles in one round of 100
+    (12480, 32, 2048, 0, False),  # the gate's one column tile: the statistic written directly
+    (190, 520, 256, 30, True),    # 64 x 64 tiles; the last block of the statistic 8 wide
+    (200, 4096, 448, 0, False),   # 64 x 64 on the whole part, 7 k steps
+    (1024, 4096, 256, 0, True),   # 128 x 128, fewer k steps than the ring has stages
+    (700, 1032, 576, 32, False),  # 128 x 128, several rounds, ragged both ways
+])
+def test_tiles_that_split_the_reduction(device, M, N, K, groups, bias):
+    """Calls too small to fill the CUs with 256 x 256 tiles, in the smaller tiles whose waves
+    split K: x and y column slices of wider buffers (y 8-byte aligned, its other columns
+    untouched), the statistic of every row, and the tiles' edges against the oracle."""
+    import torch
+
+    _say(f"linear split reduction M={M} N={N} K={K} groups={groups}")
+    xw = O.randn_bf16_bits((M, K + 16), 1400 + M)
+    w = O.randn_bf16_bits((N, K), 1500 + N, std=K ** -0.5)
+    b = O.randn_bf16_bits((N,), 1600 + N, std=0.5) if bias else None
+    big = torch.full((M, N + 12), 3.0, dtype=torch.bfloat16, device=device)
+    y, parts = L.linear(dev(xw, device)[:, 8:8 + K], dev(w, device),
+                        None if b is None else dev(b, device), out=big[:, 4:4 + N], sumsq=True,
+                        resident_groups=groups)
+    torch.cuda.synchronize()
+    rest = torch.cat([big[:, :4], big[:, 4 + N:]], dim=1).float().cpu().numpy()
+    assert np.all(rest == 3.0)
+    yb = host_bits(y)
+    rows = np.unique(np.r_[0:min(M, 70), max(0, M - 70):M])
+    check_linear(yb[rows], np.ascontiguousarray(xw[rows, 8:8 + K]), w, b, f"{M}x{N}x{K}")
+    check_partials(parts.cpu().numpy(), yb, f"{M}x{N}x{K}")
+
+
 def _random_linear_case(i):
     """Seeded draws of M (any), N (a multiple of 8), K (a multiple of 64), bias, statistic,
     the part size the tail split is planned for, and whether a workspace allows the split."""
