@@ -92,7 +92,7 @@ def check(lines, name):
                 keep.append(p)
             pending = keep
             pending.append([dst, RESULT_WAIT, f"result {sorted(dst)[0]}..", no])
-            if src != dst:
+            if src and src != dst:                # (an inline constant has no registers)
                 pending.append([src, RESULT_WAIT, f"srcC {sorted(src)[0]}..", no])
             tag = None
             waits = 1

@@ -226,6 +226,6 @@ int launch_linear_ks(const LinearParams &p, int tile, void *stream);
 int64_t linear_part_bytes(int64_t tail_tiles, int splits);          // one range: 256 KiB
 int launch_gemma_prep(const GemmaPrepParams &p, int D, void *stream);   // gemma_attn.hip
 int launch_gemma_attn(const GemmaAttnParams &p, int D, void *stream);
-int gemma_queries_per_workgroup(int D);                              // 128 (D 256), 64 (D 512)
+int gemma_queries_per_workgroup();
 
 }  // namespace ltx

@@ -25,21 +25,19 @@
 //                       32-channel block cb one 1 KB unit, lane r + 32g holding channel
 //                       32cb + r at keys 16hf + 4g + {0..3, 8..11}. Keys past T are zeros in both layouts, and
 //                       a key block's k' and v'^T are each one contiguous run of units.
-//   gemma_attn_kernel   a wave owns 32 queries over 256 channels (D = 256: the whole head;
-//                       D = 512: half of it, its partner wave the other half), four waves per
-//                       workgroup: 128 queries at D = 256, 64 at D = 512. The key blocks of
-//                       the workgroup's range are copied HBM -> LDS by the buffer-load-to-LDS
-//                       path into a ring (4 blocks at D = 256, 2 at D = 512) and read from LDS
-//                       by every wave. Per key block: S^T = K.Q'^T in fp16 products (inline,
-//                       S in VGPRs and Q' in AGPRs; at D = 512 the two halves' partial sums are
-//                       exchanged through LDS and added in a fixed order), the mask, exp2 with
-//                       each row's max fixed at its first block with an allowed key, and
-//                       O^T += V^T.P^T with v' and P in fp16 (the reference's weights are
+//   gemma_attn*_kernel  128 queries of a head per workgroup (64 at D = 512 for short prompts), a
+//                       wave 256 channels of them; the key blocks of the workgroup's range are
+//                       copied HBM -> LDS by the buffer-load-to-LDS path and read from LDS by
+//                       every wave. Per key block: S^T = K.Q'^T in fp16 products (at D = 512 the
+//                       two halves' partial sums are exchanged through LDS and added), the mask,
+//                       exp2 with each row's max fixed at its first block with an allowed key,
+//                       and O^T += V^T.P^T with v' and P in fp16 (the reference's weights are
 //                       fp32; with the max fixed a weight stays below 2^kGemmaBound). A block
 //                       whose weights would pass 2^kGemmaBound sends the workgroup to an exact
-//                       pass (online max with rescaling) over its range. O is written in
-//                       fp32, the dtype the reference's explicit path returns.
-//   gemma_combine_kernel  the long query blocks' keys run as ranges of at most 16 blocks on
+//                       pass over its range (D 256: online max with rescaling; D 512: the rows'
+//                       maxima first). O is written in fp32, the dtype the reference's explicit
+//                       path returns.
+//   gemma_combine_kernel  the long query blocks' keys run as ranges (the host's plan) on
 //                       separate workgroups, each writing unnormalised O and (max, sum); the
 //                       merge rescales and adds them.
 #include <type_traits>
@@ -234,23 +232,15 @@ __global__ __launch_bounds__(256) void gemma_prep_kernel(const GemmaPrepParams p
     else gemma_vt_block<D>(p, wg - row_wgs, tile);
 }
 // ---- attention -----------------------------------------------------------------------------
-// Geometry: a wave owns 32 queries over 256 channels of the head (D = 256: the whole head; D =
-// 512: one half, its partner wave the other). Four waves per workgroup: 128 queries at D =
-// 256, 64 at D = 512. A key block is 32 keys; its K' and V'^T operand units (D/16 and 2 * D/32
-// units of 1 KB, contiguous per block in the prologue's layout) are copied HBM -> LDS by the
-// buffer-load-to-LDS path into a ring of NS stages.
-template <int D>
-struct GemmaTile {
-    static constexpr int SPLIT = D / 256;            // waves per query group
-    static constexpr int QWG = 128 / SPLIT;          // queries per workgroup
-    static constexpr int NCW = 256 / 16;             // Q'/K' 16-channel chunks per wave
-    static constexpr int NDW = 256 / 32;             // V'^T / O 32-channel blocks per wave
-    static constexpr int KBYTES = D * 32 * 2;        // K' (or V'^T) of one key block
-    static constexpr int BLOCK = 2 * KBYTES;
-    static constexpr int NS = D == 256 ? 4 : 2;      // key blocks resident (copies in flight)
-    static constexpr int COPIES = BLOCK / 1024 / 4;  // 1 KB copies per wave per key block
-    static constexpr int XBYTES = SPLIT > 1 ? 4 * 64 * 16 * 4 : 0;   // S partial exchange
-};
+// A workgroup runs 128 queries of one head over a range of 32-key blocks, whose K' and V'^T
+// operand units (D/16 and 2 * D/32 units of 1 KB, contiguous per block in the prologue's layout)
+// are copied HBM -> LDS by the buffer-load-to-LDS path. A wave works on 256 channels: Q' and K' in
+// kNCW 16-channel chunks, V'^T and O in kNDW 32-channel blocks.
+constexpr int kGemmaQueries = 128;
+constexpr int kNCW = 256 / 16, kNDW = 256 / 32;
+// Prompts up to kGemmaShortTokens take 64 queries per workgroup at D = 512. They have one key range
+// (the host's plan splits only prompts of more than 16 key blocks).
+constexpr int kGemmaShortQueries = 64, kGemmaShortTokens = 512;
 
 // Key blocks of the query block [q0, q0 + nq): causal / window / padding bounds; a block with
 // rows inside the left padding (their rows have no allowed key) runs over all keys, those rows
@@ -265,7 +255,7 @@ __device__ __forceinline__ KeyBlocks gemma_key_blocks(const GemmaAttnParams &p, 
 
 // The fast pass keeps each row's max from its first block with an allowed key; a later block
 // whose weights would pass 2^kGemmaBound (log2 units over that max) sends the workgroup to
-// the exact pass, which rescales O and l whenever a row's max grows.
+// the exact pass.
 constexpr float kGemmaBound = 15.0f;   // the fp16 weights stay below 65504
 
 // Partial rows before query block qblk's within its head: the key ranges of the earlier query
@@ -288,167 +278,277 @@ __device__ __forceinline__ int gemma_part_offset(int T, int window, int chunk, i
     return off;
 }
 
+// The work of a workgroup: grid layer `chunk` holds every query block's chunk-th key range;
+// within a layer the heaviest (latest) query blocks come first, each across all (batch row, head)
+// pairs, so the workgroups that the dispatcher deals to the 8 XCDs in turn carry equal work.
+struct GemmaItem {
+    int chunk, nch;              // key range, of how many of its query block (chunk >= nch: none)
+    int qblk, q0, h, b, kvh, fv;
+    int kb_lo, kb_hi;            // its key blocks
+};
+__device__ __forceinline__ GemmaItem gemma_item(const GemmaAttnParams &p, int qwg) {
+    GemmaItem w;
+    const int nqb = (p.T + qwg - 1) / qwg, nbh = p.B * p.Hq, per_layer = nbh * nqb;
+    w.chunk = (int)blockIdx.x / per_layer;
+    const int rem = (int)blockIdx.x - w.chunk * per_layer;
+    w.qblk = nqb - 1 - rem / nbh;
+    const int bh = rem % nbh;
+    w.h = bh % p.Hq;
+    w.b = bh / p.Hq;
+    w.kvh = w.h / (p.Hq / p.Hkv);
+    w.q0 = w.qblk * qwg;
+    w.fv = p.first_valid[w.b];
+    const KeyBlocks kr = gemma_key_blocks(p, w.q0, qwg, w.fv);
+    w.nch = gemma_ranges(p.T, p.window, p.chunk, w.q0, qwg, w.fv);
+    w.kb_lo = kr.lo + w.chunk * p.chunk;
+    w.kb_hi = min(w.kb_lo + p.chunk - 1, kr.hi);
+    return w;
+}
+
+// The row's allowed keys as one range [k_lo, k_hi]: all keys for a row inside the left padding,
+// else causal (k <= q), past the padding (k >= fv) and inside the window (q - k < window); k_hi <=
+// T - 1 also masks the keys past T of the last block.
+__device__ __forceinline__ void gemma_allowed(const GemmaAttnParams &p, int fv, int q, int &k_lo,
+                                              int &k_hi) {
+    const bool free_row = q < fv;
+    k_lo = free_row ? 0 : max(fv, p.window > 0 ? q - p.window + 1 : 0);
+    k_hi = free_row ? p.T - 1 : min(q, p.T - 1);
+}
+
+// Mask S of key block kb (key 32 kb + 8 (i >> 2) + 4 g + (i & 3) in s[i]) and return the row's
+// max. A block inside every row's allowed range of the wave (most blocks of a causal or windowed
+// range) needs no mask: its five instructions per weight were a tenth of the block's.
+__device__ __forceinline__ float gemma_mask_max(f32x16 &s, int kb, int k_lo, int k_hi, int g) {
+    float mx = -INFINITY;
+    if (__builtin_amdgcn_ballot_w64(k_lo > 32 * kb || 32 * kb + 31 > k_hi) == 0) {
+#pragma unroll
+        for (int e = 0; e < 16; ++e) mx = fmaxf(mx, s[e]);
+    } else {
+#pragma unroll
+        for (int e = 0; e < 16; ++e) {
+            const int k = 32 * kb + 8 * (e >> 2) + 4 * g + (e & 3);
+            s[e] = ((k >= k_lo) & (k <= k_hi)) ? s[e] : -INFINITY;
+            mx = fmaxf(mx, s[e]);
+        }
+    }
+    return fmaxf(mx, xlane32(mx));
+}
+
+// fp32 weights against the row's max, their fp32 sum over this lane's keys (returned), and P in
+// fp16 for P.V (11 significant bits; the reference's explicit path multiplies fp32 weights); a row
+// with no allowed key so far has none.
+__device__ __forceinline__ float gemma_weights(const f32x16 &s, float m, u32x4 (&wh)[2]) {
+    float ts = 0.f;
+    if (m == -INFINITY) {
+        wh[0] = wh[1] = u32x4{0, 0, 0, 0};
+    } else {
+#pragma unroll
+        for (int hf = 0; hf < 2; ++hf)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const float x0 = __builtin_amdgcn_exp2f(s[8 * hf + 2 * e] - m);
+                const float x1 = __builtin_amdgcn_exp2f(s[8 * hf + 2 * e + 1] - m);
+                ts += x0 + x1;
+                wh[hf][e] = pack_f16x2(x0, x1);
+            }
+    }
+    return ts;
+}
+
+// Resource over the head's Q' rows from row `row` on (rows past T read as zeros).
 template <int D>
-__global__ __attribute__((amdgpu_flat_work_group_size(256, 256), amdgpu_waves_per_eu(1, 1)))
-void gemma_attn_kernel(const GemmaAttnParams p) {
-    using G = GemmaTile<D>;
-    constexpr int SPLIT = G::SPLIT, QWG = G::QWG, NCW = G::NCW, NDW = G::NDW, NS = G::NS;
-    __shared__ __attribute__((aligned(16))) char smem[NS * G::BLOCK + G::XBYTES];
+__device__ __forceinline__ u32x4 gemma_q_rsrc(const GemmaAttnParams &p, const GemmaItem &w, int row) {
+    return rsrc_words((const _Float16 *)p.qp + (((int64_t)w.b * p.Hq + w.h) * p.T + row) * D,
+                      (int64_t)max(0, p.T - row) * (D * 2));
+}
+
+// One lane's copies of 32 * N rows of Q' (128 channels from byte `col` of the row) into N * 8 KB
+// of LDS: rows of 256 bytes, 16-byte units XOR-swizzled by row. Read by the lanes themselves, 32
+// rows per load, a workgroup's Q' held the address unit for 4 us; so the rows arrive as runs of
+// 256 bytes. Rows past the resource arrive as zeros.
+template <int D, int N>
+__device__ __forceinline__ void gemma_copy_q(const u32x4 &rq, char *area, int lane, int col) {
+#pragma unroll
+    for (int j = 0; j < 8 * N; ++j) {
+        const int row = 4 * j + (lane >> 4);
+        copy_at(rq, (uint32_t)(uintptr_t)(lds_void *)(area + j * 1024),
+                row * (D * 2) + 16 * ((lane & 15) ^ (row & 15)), col);
+    }
+}
+__device__ __forceinline__ f16x8 gemma_q_opnd(const char *area, int row, int c, int g) {
+    return *(const __attribute__((address_space(3))) f16x8 *)(
+        (lds_void *)(area + row * 256 + 16 * ((2 * c + g) ^ (row & 15))));
+}
+
+// 32 rows x 128 channels of O^T accumulators (times `scale`) to rows of fp32 at `dst`, the first
+// `rows` of them, through the wave's own 16 KB of LDS (units swizzled by row): they leave as runs of
+// 512 bytes, where the lanes that hold them would store 32 rows per instruction.
+__device__ __forceinline__ void gemma_store_rows(char *area, const f32x16 (&o)[4], float scale, int r,
+                                                 int g, float *dst, int64_t stride, int rows) {
+#pragma unroll
+    for (int db = 0; db < 4; ++db)
+#pragma unroll
+        for (int i4 = 0; i4 < 4; ++i4) {
+            f32x4 w;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) w[e] = o[db][4 * i4 + e] * scale;
+            *(f32x4 *)(area + r * 512 + 16 * ((8 * db + 2 * i4 + g) ^ r)) = w;
+        }
+#pragma unroll
+    for (int j = 0; j < 16; ++j) {
+        const int row = 2 * j + g;
+        const f32x4 w = *(const f32x4 *)(area + row * 512 + 16 * (r ^ row));
+        if (row < rows) *(f32x4 *)(dst + row * stride + 4 * r) = w;
+    }
+}
+
+// Where a range's rows go from row `row0` of its query block on: the output, or the partials.
+struct GemmaRows {
+    float *o;                    // head's first channel
+    int64_t stride;
+    int rows;                    // rows that exist
+    float *ml;                   // partial (max, sum) or null
+};
+__device__ __forceinline__ GemmaRows gemma_rows(const GemmaAttnParams &p, const GemmaItem &w, int D,
+                                                int row0) {
+    constexpr int qwg = kGemmaQueries;
+    GemmaRows x;
+    if (w.nch > 1) {
+        const int64_t row = p.part_row0[w.b] +
+                            ((int64_t)w.h * p.part_chunks[w.b] +
+                             gemma_part_offset(p.T, p.window, p.chunk, qwg, w.fv, w.qblk) + w.chunk) *
+                                qwg + row0;
+        x = GemmaRows{p.part_o + row * D, D, qwg, p.part_ml + row * 2};
+    } else {
+        const int q = w.q0 + row0;
+        x = GemmaRows{p.out + (int64_t)w.b * p.o_bs + (int64_t)q * p.o_rs + (int64_t)w.h * D, p.o_rs,
+                      p.T - q, nullptr};
+    }
+    return x;
+}
+
+// D = 256: eight waves (two per SIMD, at most 256 registers each); a wave owns 32 queries over
+// the whole head, and a query group's two waves the even and the odd key blocks of the range,
+// merging at its end. A step is a pair of key blocks (64 KB of K' and V'^T), copied into one of
+// two stages while the other is read; one barrier per step. Two waves per SIMD overlap: alone, a
+// wave's chain S -> softmax -> P.V leaves the matrix cores idle most of the time (four waves of
+// up to 512 registers took 1.8 us per 128 queries and key block, these 0.73 us, 1.46 us a step
+// against 1.0 us of products per SIMD). What bounds a step is LDS: 256 KB of operand reads and
+// 64 KB of copies. (Two sets of waves in opposite phases, one forming S while the other ran
+// softmax and P.V, with two barriers a step, measured 0.88 us.)
+__global__ __attribute__((amdgpu_flat_work_group_size(512, 512), amdgpu_waves_per_eu(2, 2)))
+void gemma_attn256_kernel(const GemmaAttnParams p) {
+    constexpr int D = 256, QWG = kGemmaQueries, NCW = kNCW, NDW = kNDW;
+    constexpr int KBYTES = D * 32 * 2, BLOCK = 2 * KBYTES, STEP = 2 * BLOCK;
+    constexpr int COPIES = BLOCK / 1024 / 8;         // 1 KB copies per wave per key block
+    __shared__ __attribute__((aligned(16))) char smem[2 * STEP];
+    __shared__ __attribute__((aligned(16))) float xs[8 * 64 * 2];   // (max, sum) of every lane
 
     const int tid = threadIdx.x;
     const int lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int r = lane & 31, g = lane >> 5;
-    const int grp = wave / SPLIT, half = wave % SPLIT;   // query group, channel half
-    const int T = p.T;
-    const int nqb = (T + QWG - 1) / QWG;
-    // grid layer `chunk` holds every query block's chunk-th key range; within a layer the
-    // heaviest (latest) query blocks come first, each across all (batch row, head) pairs, so
-    // the workgroups that the dispatcher deals to the 8 XCDs in turn carry equal work
-    const int nbh = p.B * p.Hq;
-    const int per_layer = nbh * nqb;
-    const int chunk = (int)blockIdx.x / per_layer;
-    const int rem = (int)blockIdx.x - chunk * per_layer;
-    const int qblk = nqb - 1 - rem / nbh;
-    const int bh = rem % nbh;
-    const int h = bh % p.Hq, b = bh / p.Hq;
-    const int kvh = h / (p.Hq / p.Hkv);
-    const int q0 = qblk * QWG;
-    const int fv = p.first_valid[b];
-    const KeyBlocks kr = gemma_key_blocks(p, q0, QWG, fv);
-    const int nch = gemma_ranges(T, p.window, p.chunk, q0, QWG, fv);
-    if (chunk >= nch) return;                        // this block has fewer key ranges
-    const int kb_lo = kr.lo + chunk * p.chunk;
-    const int kb_hi = min(kb_lo + p.chunk - 1, kr.hi);
-    const int nblk = kb_hi - kb_lo + 1;
+    // query group and key blocks' parity (waves w and w + 4, on one SIMD, are a group's two)
+    const int grp = wave & 3, par = wave >> 2;
+    const GemmaItem wi = gemma_item(p, QWG);
+    if (wi.chunk >= wi.nch) return;                  // this block has fewer key ranges
+    const int T = p.T, kb_lo = wi.kb_lo, nblk = wi.kb_hi - wi.kb_lo + 1;
+    // steps of the range; of this wave (the last may hold no odd block)
+    const int nstep = (nblk + 1) / 2, mysteps = (nblk - par + 1) / 2;
 
-    // ---- copies of key blocks into the ring ---------------------------------------------
+    // ---- copies of key blocks into the stages ---------------------------------------------
     const int nkb_all = (T + 31) / 32;
-    const int64_t head_off = ((int64_t)b * p.Hkv + kvh) * nkb_all * (D * 32);   // elements
-    const u32x4 rk = rsrc_words((const bf16 *)p.kp + head_off, (int64_t)nkb_all * G::KBYTES);
-    const u32x4 rv = rsrc_words((const bf16 *)p.vt + head_off, (int64_t)nkb_all * G::KBYTES);
-    auto copy_block = [&](int i) __attribute__((always_inline)) {   // i-th block of the range
-        const int kb = kb_lo + i;
-        char *dst = smem + (i % NS) * G::BLOCK;
+    const int64_t head_off = ((int64_t)wi.b * p.Hkv + wi.kvh) * nkb_all * (D * 32);   // elements
+    const u32x4 rk = rsrc_words((const _Float16 *)p.kp + head_off, (int64_t)nkb_all * KBYTES);
+    const u32x4 rv = rsrc_words((const _Float16 *)p.vt + head_off, (int64_t)nkb_all * KBYTES);
+    auto copy_step = [&](int i) __attribute__((always_inline)) {   // i-th step of the range
+        char *dst = smem + (i & 1) * STEP;
 #pragma unroll
-        for (int j = 0; j < G::COPIES; ++j) {
-            const int u = wave * G::COPIES + j;          // 1 KB unit of the block: K' then V'^T
-            const bool isk = u < G::KBYTES / 1024;
-            const int uu = isk ? u : u - G::KBYTES / 1024;
-            copy_all(isk ? rk : rv, (uint32_t)(uintptr_t)(lds_void *)(dst + u * 1024),
-                     kb * G::KBYTES + uu * 1024 + lane * 16);
+        for (int k = 0; k < 2; ++k) {
+            if (k > 0 && i * 2 + k >= nblk) continue;        // (read by no wave)
+            const int kb = kb_lo + i * 2 + k;
+#pragma unroll
+            for (int j = 0; j < COPIES; ++j) {
+                const int u = wave * COPIES + j;             // 1 KB unit of the block: K' then V'^T
+                const bool isk = u < KBYTES / 1024;
+                const int uu = isk ? u : u - KBYTES / 1024;
+                copy_at(isk ? rk : rv,
+                        (uint32_t)(uintptr_t)(lds_void *)(dst + k * BLOCK + u * 1024), lane * 16,
+                        kb * KBYTES + uu * 1024);
+            }
         }
     };
-    // The first blocks' copies go out before the Q loads, so the two latencies overlap.
-#pragma unroll
-    for (int i = 0; i < NS - 1; ++i)
-        if (i < nblk) copy_block(i);
+    // The first step's copies go out before the Q' loads, so the two latencies overlap.
+    copy_step(0);
 
-    // ---- Q' of this wave: query q0 + 32 grp + r, channels 256 half + 16 c + 8 g .. +7 ---
-    const int q = q0 + 32 * grp + r;                 // this lane's query row
-    const int qr = min(q, T - 1);
-    const int64_t qoff = (((int64_t)b * p.Hq + h) * T + qr) * D + 256 * half + 8 * g;
+    // ---- Q' of this wave: query q0 + 32 grp + r, channels 16 c + 8 g .. +7 -----------------
+    // (through the second stage, 128 channels at a time in the wave's own 8 KB)
+    const int q = wi.q0 + 32 * grp + r;              // this lane's query row
     f16x8 qh[NCW];
+    {
+        const u32x4 rq = gemma_q_rsrc<D>(p, wi, wi.q0 + 32 * grp);
+        char *area = smem + STEP + wave * 8192;
 #pragma unroll
-    for (int c = 0; c < NCW; ++c)
-        qh[c] = __builtin_bit_cast(f16x8, ldg16((const _Float16 *)p.qp + qoff + 16 * c));
-    // Q' is only an MFMA operand: home it in AGPRs, leaving the VGPRs to S, P and operands
+        for (int ps = 0; ps < 2; ++ps) {
+            gemma_copy_q<D, 1>(rq, area, lane, 256 * ps);
+            wait_copies();
 #pragma unroll
-    for (int c = 0; c < NCW; ++c) asm volatile("" : "+a"(qh[c]));
-    // The row's allowed keys as one range [k_lo, k_hi]: all keys for a row inside the left
-    // padding, else causal (k <= q), past the padding (k >= fv) and inside the window
-    // (q - k < window); k_hi <= T - 1 also masks the keys past T of the last block.
-    const bool free_row = q < fv;
-    const int k_lo = free_row ? 0 : max(fv, p.window > 0 ? q - p.window + 1 : 0);
-    const int k_hi = free_row ? T - 1 : min(q, T - 1);
+            for (int c = 0; c < NCW / 2; ++c)
+                qh[ps * (NCW / 2) + c] = gemma_q_opnd(area, r, c, g);
+            // (in registers before the next pass's copies)
+#pragma unroll
+            for (int c = 0; c < NCW / 2; ++c) asm volatile("" : "+v"(qh[ps * (NCW / 2) + c]));
+        }
+    }
+    int k_lo, k_hi;
+    gemma_allowed(p, wi.fv, q, k_lo, k_hi);
 
     f32x16 o[NDW];
     float m, l;
-    const f32x16 zero = splat16(0.f);               // the S chains' first SrcC
-    float *xs = (float *)(smem + NS * G::BLOCK);     // [4 waves][4][64 lanes][4] partial S
     bool overflow = false;                           // some row's weights passed the bound
 
     // One pass over the range's key blocks. SAFE: the exact online softmax (O and l rescaled
-    // when a row's max grows); otherwise each row's max is fixed at its first block with an
-    // allowed key. `first`: the ring's first blocks are already on their way.
+    // when a row's max grows); otherwise each row's max is fixed at the wave's first block with
+    // an allowed key. `first`: the first step's copies are already on their way.
     auto run = [&](auto safe, bool first) __attribute__((always_inline)) {
         constexpr bool SAFE = decltype(safe)::value;
 #pragma unroll
         for (int db = 0; db < NDW; ++db) o[db] = splat16(0.f);
         m = -INFINITY;
         l = 0.f;
-        if (!first) {
-#pragma unroll
-            for (int i = 0; i < NS - 1; ++i)
-                if (i < nblk) copy_block(i);
-        }
-        for (int i = 0; i < nblk; ++i) {
-            // block i's copies have landed for this wave (later blocks' may still be in
-            // flight); after the barrier for every wave, and the stage of block i - 1 is free
-            if (i + NS - 2 < nblk) wait_copies_but<(NS - 2) * G::COPIES>();
-            else wait_copies();
+        if (!first) copy_step(0);
+        for (int i = 0; i < mysteps; ++i) {
+            // step i's copies have landed for this wave; after the barrier for every wave, and
+            // the stage of step i - 1 is free
+            wait_copies();
             __syncthreads();
-            if (i + NS - 1 < nblk) copy_block(i + NS - 1);
-            const char *Ks = smem + (i % NS) * G::BLOCK;
-            const char *Vs = Ks + G::KBYTES;
-            const int kb = kb_lo + i;
-            // S^T over this wave's channels: one chain of inline products with S in VGPRs and
-            // Q' in AGPRs (mfma_s.hpp); a product whose SrcC is the previous result issues
-            // without waiting for it
-            f32x16 s;
+            if (i + 1 < nstep) copy_step(i + 1);
+            const char *Ks = smem + (i & 1) * STEP + par * BLOCK;
+            const char *Vs = Ks + KBYTES;
+            const int kb = kb_lo + i * 2 + par;
+            auto opnd = [&](const char *base, int unit) __attribute__((always_inline)) {
+                return *(const __attribute__((address_space(3))) f16x8 *)(
+                    (lds_void *)(base + unit * 1024 + lane * 16));
+            };
+            // S^T: one chain (a product whose SrcC is the previous result issues without waiting
+            // for it)
+            constexpr int kAhead = 3;                // operands read ahead of their product
+            f32x16 s = splat16(0.f);
+            f16x8 ka[NCW];
+#pragma unroll
+            for (int c = 0; c < kAhead; ++c) ka[c] = opnd(Ks, c);
 #pragma unroll
             for (int c = 0; c < NCW; ++c) {
-                const f16x8 a = *(const __attribute__((address_space(3))) f16x8 *)(
-                    (lds_void *)(Ks + (half * NCW + c) * 1024 + lane * 16));
-                if (c == 0) s = mfma_s_first(a, qh[0], zero);
-                else mfma_s_next(s, a, qh[c]);
+                if (c + kAhead < NCW) ka[c + kAhead] = opnd(Ks, c + kAhead);
+                s = mfma32(ka[c], qh[c], s);
+                __builtin_amdgcn_sched_barrier(0);
             }
-            s_ready(s, zero);
-            if constexpr (SPLIT > 1) {
-                // the partner wave holds the other half of the channels: exchange the partial
-                // sums and add them in a fixed order, so both waves hold the same S
-                // layout [wave][i4][lane][4]: a wave's 16-byte accesses are lane-contiguous,
-                // free of bank conflicts
+            // V'^T operands (unit hf * NDW + db), the first kAhead read now: they do not depend on
+            // the softmax below, which hides their LDS round trip
+            f16x8 va[2 * NDW];
 #pragma unroll
-                for (int i4 = 0; i4 < 4; ++i4)
-                    *(f32x4 *)(xs + ((wave * 4 + i4) * 64 + lane) * 4) =
-                        f32x4{s[4 * i4], s[4 * i4 + 1], s[4 * i4 + 2], s[4 * i4 + 3]};
-                __syncthreads();
-#pragma unroll
-                for (int i4 = 0; i4 < 4; ++i4) {
-                    const f32x4 a0 = *(const f32x4 *)(xs + (((2 * grp) * 4 + i4) * 64 + lane) * 4);
-                    const f32x4 a1 = *(const f32x4 *)(xs + (((2 * grp + 1) * 4 + i4) * 64 + lane) * 4);
-#pragma unroll
-                    for (int e = 0; e < 4; ++e) s[4 * i4 + e] = a0[e] + a1[e];
-                }
-            }
-            // V'^T operands of the first key half, read now: they do not depend on the softmax
-            // below, which hides their LDS round trip (read beside the products, two at a
-            // time, each product waited for one)
-            auto v_opnd = [&](int hf, int db) __attribute__((always_inline)) {
-                return *(const __attribute__((address_space(3))) f16x8 *)(
-                    (lds_void *)(Vs + (hf * (D / 32) + half * NDW + db) * 1024 + lane * 16));
-            };
-            f16x8 va0[NDW];
-#pragma unroll
-            for (int db = 0; db < NDW; ++db) va0[db] = v_opnd(0, db);
-            // mask: key k = 32 kb + 8 (i >> 2) + 4 g + (i & 3) for query q. A block inside
-            // every row's allowed range of the wave (most blocks of a causal or windowed range)
-            // needs none: its five instructions per weight were a tenth of the block's
-            // (1024 tokens, D 256: 33.1 -> 30.8 us)
-            float mx = -INFINITY;
-            if (__builtin_amdgcn_ballot_w64(k_lo > 32 * kb || 32 * kb + 31 > k_hi) == 0) {
-#pragma unroll
-                for (int e = 0; e < 16; ++e) mx = fmaxf(mx, s[e]);
-            } else {
-#pragma unroll
-                for (int e = 0; e < 16; ++e) {
-                    const int k = 32 * kb + 8 * (e >> 2) + 4 * g + (e & 3);
-                    s[e] = ((k >= k_lo) & (k <= k_hi)) ? s[e] : -INFINITY;
-                    mx = fmaxf(mx, s[e]);
-                }
-            }
-            mx = fmaxf(mx, xlane32(mx));
+            for (int j = 0; j < kAhead; ++j) va[j] = opnd(Vs, j);
+            const float mx = gemma_mask_max(s, kb, k_lo, k_hi, g);
             if constexpr (SAFE) {
                 if (__builtin_amdgcn_ballot_w64(mx > m) != 0) {
                     const float mn = fmaxf(m, mx);
@@ -462,29 +562,460 @@ void gemma_attn_kernel(const GemmaAttnParams p) {
                 if (m == -INFINITY) m = mx;              // the row's first allowed keys
                 overflow |= mx > m + kGemmaBound;
             }
-            // fp32 weights, their fp32 row sums, and P in fp16 for P.V (11 significant bits; the
-            // reference's explicit path multiplies fp32 weights); a row with no allowed key
-            // so far has none
             u32x4 wh[2];
-            float ts = 0.f;
-            if (m == -INFINITY) {
-                wh[0] = wh[1] = u32x4{0, 0, 0, 0};
-            } else {
+            l += gemma_weights(s, m, wh);
+            // O^T += V^T.P^T; consecutive products update different accumulators (a key half over
+            // all channel blocks)
 #pragma unroll
-                for (int hf = 0; hf < 2; ++hf)
-#pragma unroll
-                    for (int e = 0; e < 4; ++e) {
-                        const float x0 = __builtin_amdgcn_exp2f(s[8 * hf + 2 * e] - m);
-                        const float x1 = __builtin_amdgcn_exp2f(s[8 * hf + 2 * e + 1] - m);
-                        ts += x0 + x1;
-                        wh[hf][e] = pack_f16x2(x0, x1);
-                    }
+            for (int j = 0; j < 2 * NDW; ++j) {
+                if (j + kAhead < 2 * NDW) va[j + kAhead] = opnd(Vs, j + kAhead);
+                o[j % NDW] = mfma32(va[j], __builtin_bit_cast(f16x8, wh[j / NDW]), o[j % NDW]);
+                __builtin_amdgcn_sched_barrier(0);
             }
-            l += ts;
-            // O^T += V^T.P^T for this wave's channels; consecutive products update different
-            // accumulators (a key half over all channel blocks). The second half's operands are
-            // read one before each product of the first half.
-            f16x8 va1[NDW];
+        }
+        if (mysteps < nstep) {
+            wait_copies();
+            __syncthreads();
+        }
+    };
+    run(std::false_type{}, true);
+    // the exact pass, for the whole workgroup, when any row outgrew its fixed max
+    if (__syncthreads_or(overflow)) run(std::true_type{}, false);
+
+    // ---- the even and odd key blocks' sums meet -------------------------------------------
+    // A group's two waves pass each other half of their O through the (free) stages: wave `par`
+    // keeps channel blocks 4 par .. 4 par + 3, both rescaled to the larger max.
+    float lt = l + xlane32(l);
+    f32x16 out[4];
+    __syncthreads();                                 // every wave is past its last step
+    {
+        float *mine = (float *)(smem + wave * 16384) + lane * 4;
+        const float *other = (const float *)(smem + (wave ^ 4) * 16384) + lane * 4;
+        auto merge = [&](auto P) __attribute__((always_inline)) {
+            constexpr int keep = decltype(P)::value * 4, pass = 4 - keep;
+#pragma unroll
+            for (int db = 0; db < 4; ++db)
+#pragma unroll
+                for (int i4 = 0; i4 < 4; ++i4) {
+                    f32x4 w;
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) w[e] = o[pass + db][4 * i4 + e];
+                    *(f32x4 *)(mine + (db * 4 + i4) * 256) = w;
+                }
+            *(f32x2 *)(xs + (wave * 64 + lane) * 2) = f32x2{m, lt};
+            __syncthreads();
+            const f32x2 ml = *(const f32x2 *)(xs + ((wave ^ 4) * 64 + lane) * 2);
+            const float mx = fmaxf(m, ml[0]);
+            // (a wave in which the row allows no key has max -inf and adds nothing)
+            const float f0 = m == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(m - mx);
+            const float f1 = ml[0] == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(ml[0] - mx);
+            m = mx;
+            lt = f0 * lt + f1 * ml[1];
+#pragma unroll
+            for (int db = 0; db < 4; ++db)
+#pragma unroll
+                for (int i4 = 0; i4 < 4; ++i4) {
+                    const f32x4 w = *(const f32x4 *)(other + (db * 4 + i4) * 256);
+#pragma unroll
+                    for (int e = 0; e < 4; ++e)
+                        out[db][4 * i4 + e] = f0 * o[keep + db][4 * i4 + e] + f1 * w[e];
+                }
+        };
+        if (par) merge(std::integral_constant<int, 1>{});
+        else merge(std::integral_constant<int, 0>{});
+    }
+
+    // ---- epilogue: O / l in fp32 (the reference's dtype here), or a range's partials ------
+    // (the lane's row again from its LDS offset, which the loops keep: carried through them, it
+    // and what hangs on it would spill)
+    int lane_again = lane * 16;
+    asm volatile("" : "+v"(lane_again));
+    const int er = (lane_again >> 4) & 31, eg = lane_again >> 9;
+    const GemmaRows to = gemma_rows(p, wi, D, 32 * grp);
+    if (to.ml && par == 0 && eg == 0) *(f32x2 *)(to.ml + er * 2) = f32x2{m, lt};
+    __syncthreads();                                 // the merge's halves are read
+    gemma_store_rows(smem + wave * 16384, out, to.ml ? 1.0f : 1.0f / lt, er, eg,
+                     to.o + 128 * par, to.stride, to.rows);
+}
+
+// D = 512: four waves (one per SIMD, up to 512 registers); a wave owns 64 queries over half of
+// the head, its mate the other half, so that each LDS operand read feeds two products (eight
+// waves of 32 queries x 256 channels read 256 KB per key block, which bound them: calls of 2 x
+// 1224 and 2 x 1472 causal tokens took 120 and 138 us, with this kernel 109 and 129; with 64
+// queries per workgroup 186 and 241). The mates split the softmax: each
+// completes S and forms P for 32 of the 64 queries, its own (local group 0; the mate's are group
+// 1), so a step passes S partials one way and P the other. Software pipeline: step i issues the
+// 32 products of S(i + 1) one at a time with a slice of the softmax of S(i) after each, then
+// P(i).V; K' runs one block ahead of V'^T, two stages of each. Two barriers a step: the first
+// publishes S(i)'s partials and the landed copies, the second P(i).
+__global__ __attribute__((amdgpu_flat_work_group_size(256, 256), amdgpu_waves_per_eu(1, 1)))
+void gemma_attn512_kernel(const GemmaAttnParams p) {
+    constexpr int D = 512, QWG = kGemmaQueries, NCW = kNCW, NDW = kNDW;
+    constexpr int KBYTES = D * 32 * 2;               // K' (or V'^T) of one key block
+    constexpr int COPIES = KBYTES / 1024 / 4;        // 1 KB copies per wave of either
+    __shared__ __attribute__((aligned(16))) char sK[2 * KBYTES];
+    __shared__ __attribute__((aligned(16))) char sV[2 * KBYTES];
+    __shared__ __attribute__((aligned(16))) float xsS[4 * 64 * 16];  // S for the mate [4][4][64][4]
+    __shared__ __attribute__((aligned(16))) uint32_t xsP[4 * 64 * 8];  // P for the mate [4][2][64][4]
+    __shared__ __attribute__((aligned(16))) float xml[4 * 64 * 2];   // (max, sum) of every lane
+
+    const int tid = threadIdx.x;
+    const int lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int r = lane & 31, g = lane >> 5;
+    const int grp = wave >> 1, half = wave & 1, mate = wave ^ 1;
+    const GemmaItem wi = gemma_item(p, QWG);
+    if (wi.chunk >= wi.nch) return;                  // this block has fewer key ranges
+    const int T = p.T, kb_lo = wi.kb_lo, nblk = wi.kb_hi - wi.kb_lo + 1;
+    const int row0 = 64 * grp;                       // the wave's queries within the block
+
+    const int nkb_all = (T + 31) / 32;
+    const int64_t head_off = ((int64_t)wi.b * p.Hkv + wi.kvh) * nkb_all * (D * 32);   // elements
+    const u32x4 rk = rsrc_words((const _Float16 *)p.kp + head_off, (int64_t)nkb_all * KBYTES);
+    const u32x4 rv = rsrc_words((const _Float16 *)p.vt + head_off, (int64_t)nkb_all * KBYTES);
+    auto copy1 = [&](const u32x4 &rs, char *stages, int i, int j) __attribute__((always_inline)) {
+        const int u = wave * COPIES + j;
+        copy_at(rs, (uint32_t)(uintptr_t)(lds_void *)(stages + (i & 1) * KBYTES + u * 1024),
+                lane * 16, (kb_lo + i) * KBYTES + u * 1024);
+    };
+    auto copy = [&](const u32x4 &rs, char *stages, int i) __attribute__((always_inline)) {
+#pragma unroll
+        for (int j = 0; j < COPIES; ++j) copy1(rs, stages, i, j);
+    };
+    // ---- Q' of this wave: local group n's query q0 + row0 + 32 (half ^ n) + r, channels
+    // 256 half + 16 c + 8 g .. +7 (through the V'^T stages, 128 channels at a time in the wave's
+    // own 16 KB; K'(0) and K'(1) follow the first half's copies)
+    f16x8 qh[2][NCW];
+    {
+        const u32x4 rq = gemma_q_rsrc<D>(p, wi, wi.q0 + row0);
+        char *area = sV + wave * 16384;
+#pragma unroll
+        for (int ps = 0; ps < 2; ++ps) {
+            gemma_copy_q<D, 2>(rq, area, lane, 512 * half + 256 * ps);
+            if (ps == 0) {
+                copy(rk, sK, 0);
+                copy(rk, sK, 1);                     // (zeros past the last key block)
+                wait_copies_but<2 * COPIES>();
+            } else {
+                wait_copies();
+            }
+#pragma unroll
+            for (int n = 0; n < 2; ++n)
+#pragma unroll
+                for (int c = 0; c < NCW / 2; ++c)
+                    qh[n][ps * (NCW / 2) + c] = gemma_q_opnd(area, 32 * (half ^ n) + r, c, g);
+#pragma unroll
+            for (int n = 0; n < 2; ++n)
+#pragma unroll
+                for (int c = 0; c < NCW / 2; ++c)
+                    asm volatile("" : "+v"(qh[n][ps * (NCW / 2) + c]));
+        }
+    }
+    const int q = wi.q0 + row0 + 32 * half + r;      // this lane's row of its own 32 queries
+    int k_lo, k_hi;
+    gemma_allowed(p, wi.fv, q, k_lo, k_hi);
+    __syncthreads();                                 // the V'^T stages are read; K'(0), K'(1) are in
+    copy(rv, sV, 0);
+
+    f32x16 o[NDW][2];
+    float m, l;
+    bool overflow = false;                           // some row's weights passed the bound
+    f32x16 sc[2];                                    // partial S of the next step's block
+    auto opnd = [&](const char *base, int unit) __attribute__((always_inline)) {
+        return *(const __attribute__((address_space(3))) f16x8 *)(
+            (lds_void *)(base + unit * 1024 + lane * 16));
+    };
+    constexpr int kAhead = 4;                        // operands read ahead of their products
+    // Partial S of block i over this wave's channels, slice(k) after product k of 32.
+    auto s_block = [&](int i, auto slice) __attribute__((always_inline)) {
+        const char *Ks = sK + (i & 1) * KBYTES;
+        f16x8 ka[NCW];
+        f32x16 sn[2];
+#pragma unroll
+        for (int c = 0; c < kAhead; ++c) ka[c] = opnd(Ks, half * NCW + c);
+#pragma unroll
+        for (int c = 0; c < NCW; ++c) {
+            if (c + kAhead < NCW) ka[c + kAhead] = opnd(Ks, half * NCW + c + kAhead);
+#pragma unroll
+            for (int n = 0; n < 2; ++n) {
+                if (c == 0) sn[n] = mfma_s_zero(ka[c], qh[n][c]);
+                else mfma_s_next_v(sn[n], ka[c], qh[n][c]);
+                slice(2 * c + n);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+        }
+        s_ready(sn[0], sn[1]);
+        sc[0] = sn[0];
+        sc[1] = sn[1];
+    };
+    // The mate's queries' partial S goes to the mate.
+    auto pass_s = [&]() __attribute__((always_inline)) {
+#pragma unroll
+        for (int i4 = 0; i4 < 4; ++i4)
+            *(f32x4 *)(xsS + ((wave * 4 + i4) * 64 + lane) * 4) =
+                f32x4{sc[1][4 * i4], sc[1][4 * i4 + 1], sc[1][4 * i4 + 2], sc[1][4 * i4 + 3]};
+    };
+
+    // A pass over the range's key blocks, each row's max fixed at its first block with an allowed
+    // key; when any row outgrows it, the rows' exact maxima, then a second pass with those.
+    m = -INFINITY;
+    auto run = [&]() __attribute__((always_inline)) {
+#pragma unroll
+        for (int db = 0; db < NDW; ++db) o[db][0] = o[db][1] = splat16(0.f);
+        l = 0.f;
+        s_block(0, [](int) {});
+        pass_s();
+        for (int i = 0; i < nblk; ++i) {
+            // This wave's share of K'(i + 1) has landed (V'^T(i)'s, issued after it, may not
+            // have); then everyone's has, S(i)'s partials are in and K' stage i is free.
+            wait_copies_but<COPIES>();
+            __syncthreads();
+            const int kb = kb_lo + i;
+            f32x4 x[4];
+#pragma unroll
+            for (int i4 = 0; i4 < 4; ++i4) x[i4] = *(const f32x4 *)(xsS + ((mate * 4 + i4) * 64 + lane) * 4);
+            f32x16 s = sc[0];
+            u32x4 wh[2];
+            // K'(i + 2) is copied between the products of S(i + 1), V'^T(i + 1) between those of
+            // P(i).V: issued together they queue, 40 to 60 cycles each (1024 padded tokens: 103
+            // -> 97 us a call). Past the range they read an empty resource, so that the waits' counts hold.
+            u32x4 rkn = rk, rvn = rv;
+            if (i + 2 >= nblk) rkn[2] = 0;
+            if (i + 1 >= nblk) rvn[2] = 0;
+            const bool more = i + 1 < nblk;
+            // A block inside every row's allowed range of the wave, whose rows all have a max:
+            // its softmax runs between the products of S(i + 1).
+            if (more &&
+                __builtin_amdgcn_ballot_w64(k_lo > 32 * kb || 32 * kb + 31 > k_hi || m == -INFINITY) == 0) {
+                float ts = 0.f, mx = -INFINITY, ex[16];
+                s_block(i + 1, [&](int k) __attribute__((always_inline)) {
+                    if ((k & 3) == 3) copy1(rkn, sK, i + 2, k >> 2);
+                    // slices 2..5 complete S, 6..9 its max, 10..25 take a weight each, and every
+                    // other of 13..27 sums and packs two
+                    if (k >= 2 && k < 6)
+                        for (int e = 0; e < 4; ++e) s[4 * (k - 2) + e] += x[k - 2][e];
+                    if (k >= 6 && k < 10)
+                        for (int e = 0; e < 4; ++e) mx = fmaxf(mx, s[4 * (k - 6) + e]);
+                    if (k >= 10 && k < 26) ex[k - 10] = __builtin_amdgcn_exp2f(s[k - 10] - m);
+                    if (k >= 13 && k < 29 && (k & 1)) {
+                        const int e = k - 13;
+                        ts += ex[e] + ex[e + 1];
+                        wh[e >> 3][(e >> 1) & 3] = pack_f16x2(ex[e], ex[e + 1]);
+                    }
+                });
+                // (each lane holds half of the row's keys: either half's overflow counts)
+                overflow |= mx > m + kGemmaBound;
+                l += ts;
+            } else {
+                copy(rkn, sK, i + 2);
+#pragma unroll
+                for (int e = 0; e < 16; ++e) s[e] += x[e >> 2][e & 3];
+                const float mx = gemma_mask_max(s, kb, k_lo, k_hi, g);
+                if (m == -INFINITY) m = mx;          // the row's first allowed keys
+                overflow |= mx > m + kGemmaBound;
+                l += gemma_weights(s, m, wh);
+                if (more) s_block(i + 1, [](int) {});
+            }
+#pragma unroll
+            for (int hf = 0; hf < 2; ++hf) *(u32x4 *)(xsP + ((wave * 2 + hf) * 64 + lane) * 4) = wh[hf];
+            const char *Vs = sV + (i & 1) * KBYTES;
+            auto v_opnd = [&](int j) __attribute__((always_inline)) {
+                return opnd(Vs, (j / NDW) * (D / 32) + half * NDW + j % NDW);
+            };
+            f16x8 va[2 * NDW];
+            wait_copies_but<COPIES>();
+            __syncthreads();     // P(i) and V'^T(i) are in; S(i)'s partials are read
+            if (more) pass_s();
+            u32x4 wo[2];
+#pragma unroll
+            for (int hf = 0; hf < 2; ++hf) wo[hf] = *(const u32x4 *)(xsP + ((mate * 2 + hf) * 64 + lane) * 4);
+#pragma unroll
+            for (int j = 0; j < kAhead; ++j) va[j] = v_opnd(j);
+#pragma unroll
+            for (int j = 0; j < 2 * NDW; ++j) {
+                if (j + kAhead < 2 * NDW) va[j + kAhead] = v_opnd(j + kAhead);
+                o[j % NDW][0] = mfma32(va[j], __builtin_bit_cast(f16x8, wh[j / NDW]), o[j % NDW][0]);
+                o[j % NDW][1] = mfma32(va[j], __builtin_bit_cast(f16x8, wo[j / NDW]), o[j % NDW][1]);
+                if (j & 1) copy1(rvn, sV, i + 1, j >> 1);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+        }
+        wait_copies();
+    };
+    run();
+    if (__syncthreads_or(overflow)) {
+        m = -INFINITY;
+        for (int i = 0; i < nblk; ++i) {
+            __syncthreads();
+            copy(rk, sK, i);
+            wait_copies();
+            __syncthreads();
+            s_block(i, [](int) {});
+            pass_s();
+            __syncthreads();
+            f32x16 s = sc[0];
+#pragma unroll
+            for (int i4 = 0; i4 < 4; ++i4) {
+                const f32x4 x = *(const f32x4 *)(xsS + ((mate * 4 + i4) * 64 + lane) * 4);
+#pragma unroll
+                for (int e = 0; e < 4; ++e) s[4 * i4 + e] += x[e];
+            }
+            m = fmaxf(m, gemma_mask_max(s, kb_lo + i, k_lo, k_hi, g));
+        }
+        __syncthreads();
+        copy(rk, sK, 0);
+        if (nblk > 1) copy(rk, sK, 1);
+        copy(rv, sV, 0);
+        wait_copies();
+        __syncthreads();
+        run();
+    }
+
+    // ---- epilogue: O / l in fp32 (the reference's dtype here), or a range's partials ------
+    // (the lane's row again from its LDS offset, as in the D 256 kernel)
+    int lane_again = lane * 16;
+    asm volatile("" : "+v"(lane_again));
+    const int er = (lane_again >> 4) & 31, eg = lane_again >> 9, el = lane_again >> 4;
+    const float lt = l + xlane32(l);
+    *(f32x2 *)(xml + (wave * 64 + el) * 2) = f32x2{m, lt};
+    __syncthreads();                                 // (also: every wave is past its last V'^T)
+    char *area = (wave < 2 ? sK : sV) + (wave & 1) * 16384;
+    const GemmaRows to = gemma_rows(p, wi, D, row0);
+    if (to.ml && eg == 0) *(f32x2 *)(to.ml + (32 * half + er) * 2) = f32x2{m, lt};
+#pragma unroll
+    for (int n = 0; n < 2; ++n) {
+        const int first = 32 * (half ^ n);           // of the group's 32 queries, within the 64
+        asm volatile("" ::: "memory");               // (the sum from LDS when it is needed)
+        const float sum = xml[((n == 0 ? wave : mate) * 64 + el) * 2 + 1];
+        const float scale = to.ml ? 1.0f : 1.0f / sum;
+#pragma unroll
+        for (int d0 = 0; d0 < NDW; d0 += 4) {
+            f32x16 out[4];
+#pragma unroll
+            for (int db = 0; db < 4; ++db) {
+                // (whole in its registers until here: taken apart earlier, it was moved around)
+                asm volatile("" : "+a"(o[d0 + db][n]));
+                out[db] = o[d0 + db][n];
+            }
+            gemma_store_rows(area, out, scale, er, eg, to.o + first * to.stride + 256 * half + 32 * d0,
+                             to.stride, to.rows - first);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+    }
+}
+
+// D = 512, short prompts: 64 queries per workgroup, a wave 32 of them over half of the head (its
+// partner wave the other half), one key block at a time, no key ranges. Twice as many
+// workgroups, each with half of the 128-query kernel's start and epilogue, which bound a prompt of
+// a few blocks: 72 / 144 / 256 / 512 tokens 23.4 / 26.1 / 33.9 / 53.2 us a call against 26.9 /
+// 28.8 / 37.5 / 54.7. From 544 tokens on (a split plan's first) the other kernel is the faster.
+__global__ __attribute__((amdgpu_flat_work_group_size(256, 256), amdgpu_waves_per_eu(1, 1)))
+void gemma_attn512_short_kernel(const GemmaAttnParams p) {
+    constexpr int D = 512, QWG = kGemmaShortQueries, NCW = kNCW, NDW = kNDW;
+    constexpr int KBYTES = D * 32 * 2, BLOCK = 2 * KBYTES, COPIES = BLOCK / 1024 / 4;
+    __shared__ __attribute__((aligned(16))) char smem[2 * BLOCK];
+    __shared__ __attribute__((aligned(16))) float xs[4 * 64 * 16];   // partial S [4][4][64][4]
+
+    const int tid = threadIdx.x;
+    const int lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int r = lane & 31, g = lane >> 5;
+    const int grp = wave >> 1, half = wave & 1;
+    const GemmaItem wi = gemma_item(p, QWG);
+    const int T = p.T, kb_lo = wi.kb_lo, nblk = wi.kb_hi - wi.kb_lo + 1;
+    const int nkb_all = (T + 31) / 32;
+    const int64_t head_off = ((int64_t)wi.b * p.Hkv + wi.kvh) * nkb_all * (D * 32);   // elements
+    const u32x4 rk = rsrc_words((const _Float16 *)p.kp + head_off, (int64_t)nkb_all * KBYTES);
+    const u32x4 rv = rsrc_words((const _Float16 *)p.vt + head_off, (int64_t)nkb_all * KBYTES);
+    auto copy_block = [&](int i) __attribute__((always_inline)) {   // i-th block of the range
+        char *dst = smem + (i & 1) * BLOCK;
+#pragma unroll
+        for (int j = 0; j < COPIES; ++j) {
+            const int u = wave * COPIES + j;         // 1 KB unit of the block: K' then V'^T
+            const bool isk = wave < 2;
+            copy_at(isk ? rk : rv, (uint32_t)(uintptr_t)(lds_void *)(dst + u * 1024), lane * 16,
+                    (kb_lo + i) * KBYTES + (isk ? u : u - KBYTES / 1024) * 1024);
+        }
+    };
+    copy_block(0);
+
+    // Q' of this wave (through the wave's own 16 KB of the second stage)
+    f16x8 qh[NCW];
+    {
+        const u32x4 rq = gemma_q_rsrc<D>(p, wi, wi.q0 + 32 * grp);
+        char *area = smem + BLOCK + wave * 16384;
+#pragma unroll
+        for (int ps = 0; ps < 2; ++ps)
+            gemma_copy_q<D, 1>(rq, area + ps * 8192, lane, 512 * half + 256 * ps);
+        wait_copies();
+#pragma unroll
+        for (int c = 0; c < NCW; ++c)
+            qh[c] = gemma_q_opnd(area + (c / 8) * 8192, r, c % 8, g);
+        // Q' is only an MFMA operand: home it in AGPRs, leaving the VGPRs to S, P and operands
+#pragma unroll
+        for (int c = 0; c < NCW; ++c) asm volatile("" : "+a"(qh[c]));
+    }
+    const int q = wi.q0 + 32 * grp + r;              // this lane's query row
+    int k_lo, k_hi;
+    gemma_allowed(p, wi.fv, q, k_lo, k_hi);
+
+    f32x16 o[NDW];
+    float m = -INFINITY, l;
+    const f32x16 zero = splat16(0.f);                // the S chains' first SrcC
+    bool overflow = false;                           // some row's weights passed the bound
+    auto opnd = [&](const char *base, int unit) __attribute__((always_inline)) {
+        return *(const __attribute__((address_space(3))) f16x8 *)(
+            (lds_void *)(base + unit * 1024 + lane * 16));
+    };
+    // Block i: landed and published, the next block's copies issued; S of this wave's rows, the
+    // partner's half of the channels added.
+    auto s_block = [&](int i) __attribute__((always_inline)) {
+        wait_copies();
+        __syncthreads();
+        if (i + 1 < nblk) copy_block(i + 1);
+        const char *Ks = smem + (i & 1) * BLOCK;
+        f32x16 s;
+#pragma unroll
+        for (int c = 0; c < NCW; ++c) {
+            const f16x8 a = opnd(Ks, half * NCW + c);
+            if (c == 0) s = mfma_s_first(a, qh[0], zero);
+            else mfma_s_next(s, a, qh[c]);
+        }
+        s_ready(s, zero);
+        // (a wave's 16-byte accesses are lane-contiguous, free of bank conflicts)
+#pragma unroll
+        for (int i4 = 0; i4 < 4; ++i4)
+            *(f32x4 *)(xs + ((wave * 4 + i4) * 64 + lane) * 4) =
+                f32x4{s[4 * i4], s[4 * i4 + 1], s[4 * i4 + 2], s[4 * i4 + 3]};
+        __syncthreads();
+#pragma unroll
+        for (int i4 = 0; i4 < 4; ++i4) {
+            const f32x4 x = *(const f32x4 *)(xs + (((wave ^ 1) * 4 + i4) * 64 + lane) * 4);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) s[4 * i4 + e] += x[e];
+        }
+        return s;
+    };
+    // Passes as in the 128-query kernel.
+    auto run = [&]() __attribute__((always_inline)) {
+#pragma unroll
+        for (int db = 0; db < NDW; ++db) o[db] = splat16(0.f);
+        l = 0.f;
+        for (int i = 0; i < nblk; ++i) {
+            f32x16 s = s_block(i);
+            const char *Vs = smem + (i & 1) * BLOCK + KBYTES;
+            auto v_opnd = [&](int hf, int db) __attribute__((always_inline)) {
+                return opnd(Vs, hf * (D / 32) + half * NDW + db);
+            };
+            // the first key half's operands: their LDS round trip passes behind the softmax
+            f16x8 va0[NDW], va1[NDW];
+#pragma unroll
+            for (int db = 0; db < NDW; ++db) va0[db] = v_opnd(0, db);
+            const float mx = gemma_mask_max(s, kb_lo + i, k_lo, k_hi, g);
+            if (m == -INFINITY) m = mx;              // the row's first allowed keys
+            overflow |= mx > m + kGemmaBound;
+            u32x4 wh[2];
+            l += gemma_weights(s, m, wh);
 #pragma unroll
             for (int db = 0; db < NDW; ++db) {
                 va1[db] = v_opnd(1, db);
@@ -496,46 +1027,33 @@ void gemma_attn_kernel(const GemmaAttnParams p) {
                 o[db] = mfma32(va1[db], __builtin_bit_cast(f16x8, wh[1]), o[db]);
         }
     };
-    run(std::false_type{}, true);
-    // the exact pass, for the whole workgroup, when any row outgrew its fixed max
-    if (__syncthreads_or(overflow)) run(std::true_type{}, false);
-
-    // ---- epilogue: O / l in fp32 (the reference's dtype here), this wave's channels ------
-    const float lt = l + xlane32(l);
-    if (nch > 1) {
-        // one key range of several: unnormalised O, then (max, sum) per row, for the combine
-        const int64_t row = p.part_row0[b] +
-                            ((int64_t)h * p.part_chunks[b] +
-                             gemma_part_offset(T, p.window, p.chunk, QWG, fv, qblk) + chunk) * QWG +
-                            32 * grp + r;
-        float *po = p.part_o + row * D + 256 * half;
-#pragma unroll
-        for (int db = 0; db < NDW; ++db)
-#pragma unroll
-            for (int i4 = 0; i4 < 4; ++i4) {
-                f32x4 w;
-#pragma unroll
-                for (int e = 0; e < 4; ++e) w[e] = o[db][4 * i4 + e];
-                *(f32x4 *)(po + 32 * db + 8 * i4 + 4 * g) = w;
-            }
-        if (half == 0 && g == 0) {
-            p.part_ml[row * 2] = m;
-            p.part_ml[row * 2 + 1] = lt;
+    run();
+    if (__syncthreads_or(overflow)) {
+        m = -INFINITY;
+        copy_block(0);
+        for (int i = 0; i < nblk; ++i) {
+            f32x16 s = s_block(i);
+            m = fmaxf(m, gemma_mask_max(s, kb_lo + i, k_lo, k_hi, g));
         }
-        return;
+        __syncthreads();
+        copy_block(0);
+        run();
     }
-    if (q < T) {
-        const float inv = 1.0f / lt;
-        float *Ob = p.out + (int64_t)b * p.o_bs + (int64_t)q * p.o_rs + (int64_t)h * D + 256 * half;
+
+    const float lt = l + xlane32(l);
+    __syncthreads();                                 // every wave is past its last V'^T
+    const GemmaRows to = gemma_rows(p, wi, D, 32 * grp);
 #pragma unroll
-        for (int db = 0; db < NDW; ++db)
+    for (int d0 = 0; d0 < NDW; d0 += 4) {
+        f32x16 out[4];
 #pragma unroll
-            for (int i4 = 0; i4 < 4; ++i4) {
-                f32x4 w;
-#pragma unroll
-                for (int e = 0; e < 4; ++e) w[e] = o[db][4 * i4 + e] * inv;
-                *(f32x4 *)(Ob + 32 * db + 8 * i4 + 4 * g) = w;
-            }
+        for (int db = 0; db < 4; ++db) {
+            asm volatile("" : "+a"(o[d0 + db]));
+            out[db] = o[d0 + db];
+        }
+        gemma_store_rows(smem + (2 * wave + d0 / 4) * 16384, out, 1.0f / lt, r, g,
+                         to.o + 256 * half + 32 * d0, to.stride, to.rows);
+        __builtin_amdgcn_sched_barrier(0);
     }
 }
 
@@ -551,7 +1069,7 @@ constexpr int kCombineRows = 4;
 template <int D, int N>
 __device__ __forceinline__ void gemma_merge_rows(const GemmaAttnParams &p, int64_t row0, int ch,
                                                  int q, float *out) {
-    constexpr int QWG = GemmaTile<D>::QWG;
+    constexpr int QWG = kGemmaQueries;
     constexpr int RPW = 256 / (D / 4);
     constexpr int PASS = N <= 2 ? kCombineRows : N <= 4 ? kCombineRows / 2 : 1;
 #pragma unroll
@@ -593,7 +1111,7 @@ __device__ __forceinline__ void gemma_merge_rows(const GemmaAttnParams &p, int64
 
 template <int D>
 __global__ __launch_bounds__(256) void gemma_combine_kernel(const GemmaAttnParams p) {
-    constexpr int QWG = GemmaTile<D>::QWG;
+    constexpr int QWG = kGemmaQueries;
     constexpr int U = D / 4;                        // threads per row
     constexpr int RPW = 256 / U;                    // rows per pass of the workgroup
     constexpr int WG_PER_QB = QWG / (RPW * kCombineRows);
@@ -644,22 +1162,24 @@ int launch_gemma_prep(const GemmaPrepParams &p, int D, void *stream) {
 }
 
 int launch_gemma_attn(const GemmaAttnParams &p, int D, void *stream) {
-    const int qwg = D == 512 ? GemmaTile<512>::QWG : GemmaTile<256>::QWG;
-    const int64_t per_layer = (int64_t)p.B * p.Hq * ((p.T + qwg - 1) / qwg);
-    const dim3 grid((unsigned)(per_layer * p.nch_max)), block(256);
+    const int64_t per_layer = (int64_t)p.B * p.Hq * ((p.T + kGemmaQueries - 1) / kGemmaQueries);
+    const dim3 grid((unsigned)(per_layer * p.nch_max));
     hipStream_t st = (hipStream_t)stream;
-    if (D == 512) hipLaunchKernelGGL(gemma_attn_kernel<512>, grid, block, 0, st, p);
-    else hipLaunchKernelGGL(gemma_attn_kernel<256>, grid, block, 0, st, p);
+    if (D == 512 && p.T <= kGemmaShortTokens)
+        hipLaunchKernelGGL(gemma_attn512_short_kernel,
+                           dim3((unsigned)((int64_t)p.B * p.Hq *
+                                           ((p.T + kGemmaShortQueries - 1) / kGemmaShortQueries))),
+                           dim3(256), 0, st, p);
+    else if (D == 512) hipLaunchKernelGGL(gemma_attn512_kernel, grid, dim3(256), 0, st, p);
+    else hipLaunchKernelGGL(gemma_attn256_kernel, grid, dim3(512), 0, st, p);
     if (p.nch_max > 1) {
-        const dim3 cgrid((unsigned)(per_layer * qwg / (256 / (D / 4) * kCombineRows)));
-        if (D == 512) hipLaunchKernelGGL(gemma_combine_kernel<512>, cgrid, block, 0, st, p);
-        else hipLaunchKernelGGL(gemma_combine_kernel<256>, cgrid, block, 0, st, p);
+        const dim3 cgrid((unsigned)(per_layer * kGemmaQueries / (256 / (D / 4) * kCombineRows)));
+        if (D == 512) hipLaunchKernelGGL(gemma_combine_kernel<512>, cgrid, dim3(256), 0, st, p);
+        else hipLaunchKernelGGL(gemma_combine_kernel<256>, cgrid, dim3(256), 0, st, p);
     }
     return (int)hipGetLastError();
 }
 
-int gemma_queries_per_workgroup(int D) {
-    return D == 512 ? GemmaTile<512>::QWG : GemmaTile<256>::QWG;
-}
+int gemma_queries_per_workgroup() { return kGemmaQueries; }
 
 }  // namespace ltx

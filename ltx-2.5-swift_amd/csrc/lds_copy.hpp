@@ -37,6 +37,17 @@ __device__ __forceinline__ void copy_all(u32x4 rs, uint32_t lds_byte, int voff) 
         : "m0", "memory");
 }
 
+// The same with part of the offset, `soff`, uniform.
+__device__ __forceinline__ void copy_at(u32x4 rs, uint32_t lds_byte, int voff, int soff) {
+    asm volatile(
+        "s_mov_b32 m0, %0\n\t"
+        "s_nop 0\n\t"
+        "buffer_load_dwordx4 %1, %2, %3 offen lds"
+        :
+        : "s"(lds_byte), "v"(voff), "s"(rs), "s"(soff)
+        : "m0", "memory");
+}
+
 // Buffer resource words over [base, base + bytes) (raw, 32-bit format): loads past the end
 // return zero.
 __device__ __forceinline__ u32x4 rsrc_words(const void *base, int64_t bytes) {

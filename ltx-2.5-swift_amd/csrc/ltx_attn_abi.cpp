@@ -377,16 +377,73 @@ struct GemmaPlan {
     int32_t part_chunks[ltx::kMaxBatch] = {}; // split ranges per head of each batch row
 };
 
-// Key blocks (32 keys) per range of a Gemma query block. The latest query blocks of a causal
-// layer walk every key block while the earliest walk a few; ranges of at most 16 blocks spread
-// the long ones over several CUs at the price of fp32 partials and a merge. Measured at 1024
-// tokens (MI355X, attention + merge): ranges of 16 blocks 45 + 7 us (D 256, 128-query
-// workgroups) and 79 + 11 us (D 512, 64-query workgroups), of 8 blocks 53 + 10 and 99 + 17 us.
-// Longer prompts take longer ranges, so that a query block never has more than the merge's
-// kGemmaMaxChunks.
+// Partials (rows of D + 2 floats) of a Gemma call whose query blocks of qwg queries run their
+// keys in ranges of `chunk` 32-key blocks: kept for the ranges of query blocks that have more
+// than one, per batch row (its padding decides which blocks split), head-major. Also the call's
+// key blocks over all its workgroups, its longest range and its workgroups.
+struct GemmaRanges {
+    int64_t rows = 0, blocks = 0, groups = 0;
+    int32_t longest = 0;
+};
+GemmaRanges gemma_ranges_of(const ltx_gemma_attn_args *a, int qwg, int chunk, int64_t *row0,
+                            int32_t *chunks) {
+    GemmaRanges g;
+    for (int b = 0; b < a->B; ++b) {
+        const int fv = a->first_valid ? a->first_valid[b] : 0;
+        int split = 0;
+        for (int q0 = 0; q0 < a->T; q0 += qwg) {
+            const int n = ltx::gemma_ranges(a->T, a->window, chunk, q0, qwg, fv);
+            const int len = ltx::gemma_key_hi(a->T, q0, qwg, fv) -
+                            ltx::gemma_key_lo(q0, fv, a->window) + 1;
+            if (n > 1) split += n;
+            g.blocks += (int64_t)a->Hq * len;
+            g.groups += (int64_t)a->Hq * n;
+            g.longest = std::max(g.longest, std::min(len, chunk));
+        }
+        if (row0) row0[b] = g.rows;
+        if (chunks) chunks[b] = split;
+        g.rows += (int64_t)a->Hq * split * qwg;
+    }
+    return g;
+}
+
+// The workspace a call asks for holds the partials of 64-query (D 512) or 128-query (D 256)
+// blocks in ranges of 16 key blocks (longer for prompts past 128 key blocks, so that a query
+// block never has more than the merge's kGemmaMaxChunks).
 int32_t gemma_chunk_blocks(int32_t T) {
     const int nkb = (T + 31) / 32;
     return std::max(std::min(nkb, 16), (nkb + ltx::kGemmaMaxChunks - 1) / ltx::kGemmaMaxChunks);
+}
+
+// The range length a call runs with: the cheapest, by an estimate in us, of the even lengths
+// whose partials fit in `rows`. A range spreads a long query block over several CUs at the price
+// of fp32 partials (written and read back at about 5 TB/s) and a merge launch; one workgroup runs
+// per CU, the longest ranges first. A block takes a workgroup 0.75 us at D 256 (two at a time) and
+// 1.9 us at D 512, its start and epilogue about 8 us. Measured at 1024 tokens, attention + merge,
+// one range / two / three: D 256 causal 36 / 27 + 7 / 25 + 9 us; D 512 over all keys 86 / 54 +
+// 16 / 77 + 21 us.
+int32_t gemma_run_chunk(const ltx_gemma_attn_args *a, int64_t rows) {
+    const int nkb = (a->T + 31) / 32, qwg = ltx::gemma_queries_per_workgroup();
+    const int least = (nkb + ltx::kGemmaMaxChunks - 1) / ltx::kGemmaMaxChunks;
+    const double block_us = a->D == 512 ? 1.9 : 0.75, start_us = 8.0, merge_us = 4.0;
+    constexpr int kGroups = 256;
+    const int step = std::max(2, (nkb / 16) & ~1);
+    int32_t best = nkb;
+    double best_us = 0.0;
+    for (int c = nkb; c >= std::max(least, 4); c = (c - 1) / step * step) {
+        const GemmaRanges g = gemma_ranges_of(a, qwg, c, nullptr, nullptr);
+        if (g.rows > rows) continue;
+        const double avg = (g.blocks * block_us + g.groups * start_us) / kGroups;
+        const double us =
+            std::max(g.longest * block_us + start_us, avg + (g.groups > kGroups ? 0.25 : 0.0) *
+                                                                g.longest * block_us) +
+            (g.rows ? merge_us + (double)g.rows * a->D * 8 / 5e6 : 0.0);
+        if (best_us == 0.0 || us < best_us) {
+            best = c;
+            best_us = us;
+        }
+    }
+    return best;
 }
 
 ltx_attn_status gemma_plan(const ltx_gemma_attn_args *a, GemmaPlan *pl) {
@@ -437,29 +494,17 @@ ltx_attn_status gemma_plan(const ltx_gemma_attn_args *a, GemmaPlan *pl) {
     pl->off_k = align_up(qn, 256);
     pl->off_v = pl->off_k + align_up(kn, 256);
     pl->bytes = pl->off_v + align_up(kn, 256);
-    const int qwg = ltx::gemma_queries_per_workgroup(a->D);
-    const int nkb = (a->T + 31) / 32, nqb = (a->T + qwg - 1) / qwg;
-    pl->chunk = gemma_chunk_blocks(a->T);
-    pl->nch_max = (nkb + pl->chunk - 1) / pl->chunk;
-    if (pl->nch_max > 1) {
-        // partials only for the ranges of query blocks that have more than one, laid out per
-        // batch row (its padding decides which blocks split), head-major
-        size_t rows = 0;
-        for (int b = 0; b < a->B; ++b) {
-            const int fv = a->first_valid ? a->first_valid[b] : 0;
-            int chunks = 0;
-            for (int j = 0; j < nqb; ++j) {
-                const int n = ltx::gemma_ranges(a->T, a->window, pl->chunk, j * qwg, qwg, fv);
-                if (n > 1) chunks += n;
-            }
-            pl->part_row0[b] = (int64_t)rows;
-            pl->part_chunks[b] = chunks;
-            rows += (size_t)a->Hq * chunks * qwg;
-        }
+    const int64_t rows =
+        gemma_ranges_of(a, a->D == 512 ? 64 : 128, gemma_chunk_blocks(a->T), nullptr, nullptr).rows;
+    if ((a->T + 31) / 32 > gemma_chunk_blocks(a->T)) {
         pl->off_po = pl->bytes;
-        pl->off_pml = pl->off_po + align_up(rows * D * 4, 256);
-        pl->bytes = pl->off_pml + align_up(rows * 2 * 4, 256);
+        pl->off_pml = pl->off_po + align_up((size_t)rows * D * 4, 256);
+        pl->bytes = pl->off_pml + align_up((size_t)rows * 2 * 4, 256);
     }
+    pl->chunk = gemma_run_chunk(a, rows);
+    gemma_ranges_of(a, ltx::gemma_queries_per_workgroup(), pl->chunk, pl->part_row0,
+                    pl->part_chunks);
+    pl->nch_max = ((a->T + 31) / 32 + pl->chunk - 1) / pl->chunk;
     return LTX_ATTN_OK;
 }
 

@@ -49,6 +49,20 @@ __device__ __forceinline__ void mfma_s_next(f32x16 &acc, f16x8 a, f16x8 b) {
     asm("; mfma_s %0 src %0\n\tv_mfma_f32_32x32x16_f16 %0, %1, %2, %0"
         : "+v"(acc) : "v"(a), "a"(b));
 }
+// And with Q in VGPRs too (a kernel whose O fills the AGPRs), the chain starting from zero.
+__device__ __forceinline__ f32x16 mfma_s_zero(f16x8 a, f16x8 b) {
+    f32x16 d;
+    asm("; mfma_s %0 src 0\n\ts_nop 1\n\tv_mfma_f32_32x32x16_f16 %0, %1, %2, 0"
+        : "=&v"(d) : "v"(a), "v"(b));
+    return d;
+}
+__device__ __forceinline__ void mfma_s_next_v(f32x16 &acc, f16x8 a, f16x8 b) {
+    asm("; mfma_s %0 src %0\n\tv_mfma_f32_32x32x16_f16 %0, %1, %2, %0"
+        : "+v"(acc) : "v"(a), "v"(b));
+}
+__device__ __forceinline__ void s_ready(f32x16 &x, f32x16 &y) {
+    asm volatile("; s_ready %0 %1\n\ts_nop 7\n\ts_nop 7\n\ts_nop 3" : "+v"(x), "+v"(y));
+}
 __device__ __forceinline__ void s_ready(f32x16 &x, const f32x16 &c0) {
     asm volatile("; s_ready %0\n\ts_nop 7\n\ts_nop 7\n\ts_nop 3" : "+v"(x) : "v"(c0));
 }

@@ -147,3 +147,34 @@ def test_gemma_attention(device, name):
         assert c["max_abs"] <= 2e-2, c
     if ref is not None:
         assert c["rel_rms"] <= max(r["rel_rms"], 2.5e-3) * 1.25, (c, r)
+
+
+# Where the kernels change: one key block, an odd last block (D 256 takes them in pairs), rows of a
+# workgroup past T, the longest prompt of the 64-query D 512 kernel and the shortest of the
+# 128-query one, and the exact pass of each (large logits), with and without key ranges.
+EDGES = {
+    "sliding_T28": dict(T=28, kind="sliding", fv=[0]),
+    "sliding_T92_B2": dict(T=92, kind="sliding", fv=[0, 60]),
+    "sliding_T132": dict(T=132, kind="sliding", fv=[0]),
+    "full_T28": dict(T=28, kind="full", fv=[0]),
+    "full_T512_pad300": dict(T=512, kind="full", fv=[300]),
+    "full_T516_B2": dict(T=516, kind="full", fv=[0, 515]),
+    "full_T640": dict(T=640, kind="full", fv=[0]),
+    "sliding_T92_large": dict(T=92, kind="sliding", fv=[0], wk_mean=3.0),
+    "full_T132_large": dict(T=132, kind="full", fv=[0], wk_mean=3.0),
+    "full_T772_pad40_large": dict(T=772, kind="full", fv=[40], wk_mean=3.0),
+}
+
+
+@pytest.mark.parametrize("name", sorted(EDGES))
+def test_gemma_kernel_edges(device, name):
+    _say(f"gemma {name}")
+    case = dict(EDGES[name], B=len(EDGES[name]["fv"]), seed=0x5EED + 900 + len(name))
+    got, truth, ref = _run(device, case)
+    c, r = O.compare(got, truth), O.compare(ref, truth)
+    _say(f"  relRMS {c['rel_rms']:.3e} maxAbs {c['max_abs']:.3e} "
+         f"(reference arithmetic relRMS {r['rel_rms']:.3e})")
+    # the bounds of test_gemma_attention; large logits take only the relative one
+    if "wk_mean" not in case:
+        assert c["rel_rms"] <= 5e-3 and c["max_abs"] <= 2e-2, c
+    assert c["rel_rms"] <= max(r["rel_rms"], 2.5e-3) * 1.25, (c, r)
