@@ -656,26 +656,33 @@ __device__ __forceinline__ void qk_prep_rows(const PrepParams &p, int blk) {
     }
 }
 
-// One launch for one row set, or for two (the Q statistic and the K prologue of one call):
-// the first blocks_a workgroups take set a, the rest set b.
+// The statistic alone from a projection's partial sums: one thread per token row, the partials
+// added in order, the same formula as above.
+template <int D>
+__device__ __forceinline__ void partial_rows(const PrepParams &p, int blk) {
+    const int64_t row = (int64_t)blk * NT + threadIdx.x;
+    if (row >= (int64_t)p.B * p.L) return;
+    const float *parts = p.sumsq + row * p.ss_rs;
+    float tot = 0.f;
+#pragma unroll 8
+    for (int j = 0; j < p.ss_blocks; ++j) tot += parts[j];
+    p.rstd[row] = 1.0f / sqrtf(tot / (float)(p.H * D) + p.eps);
+}
+
+// One launch for one row set, or for two (a call's Q and K passes): the first blocks_a workgroups
+// take set a, the rest set b. A statistic given as partials is a set too: as a launch of its own it
+// took 4.8 us of kernel for 3120 rows, most of it start and end, and a gap in front of the next
+// launch (3120 text-cross queries 75.6 -> 70.4 us a call, 3120-token self-attention 182 -> 177;
+// with both statistics given, 101 queries over 12480 keys, 50.1 -> 46.8).
 template <int D, int UPL>
 __global__ __launch_bounds__(NT) void qk_prep_kernel(const PrepParams a, const PrepParams b,
                                                      const int blocks_a) {
-    if ((int)blockIdx.x < blocks_a) qk_prep_rows<D, UPL>(a, blockIdx.x);
-    else qk_prep_rows<D, UPL>(b, blockIdx.x - blocks_a);
-}
-
-// ------------------------------------------------------------------------------------------
-// RMS statistic from the projection's partial sums of squares: one thread per token row,
-// partials added in order, the same formula as the prologue's.
-// ------------------------------------------------------------------------------------------
-__global__ __launch_bounds__(256) void rstd_kernel(const RstdParams p) {
-    const int row = blockIdx.x * 256 + threadIdx.x;
-    if (row >= p.rows) return;
-    const float *parts = p.sumsq + (int64_t)row * p.rs;
-    float tot = 0.f;
-    for (int j = 0; j < p.blocks; ++j) tot += parts[j];
-    p.rstd[row] = 1.0f / sqrtf(tot / (float)p.n + p.eps);
+    const bool first = (int)blockIdx.x < blocks_a;
+    const PrepParams &p = first ? a : b;
+    const int blk = first ? blockIdx.x : blockIdx.x - blocks_a;
+    if (p.sumsq && !p.out) partial_rows<D>(p, blk);
+    else if (first) qk_prep_rows<D, UPL>(a, blk);
+    else qk_prep_rows<D, UPL>(b, blk);
 }
 
 // ------------------------------------------------------------------------------------------
@@ -785,12 +792,6 @@ int launch_fmha(const FmhaParams &p, int D, int kind, void *stream) {
     return (int)hipGetLastError();
 }
 
-int launch_rstd(const RstdParams &p, void *stream) {
-    const dim3 grid((unsigned)((p.rows + 255) / 256)), block(256);
-    hipLaunchKernelGGL(rstd_kernel, grid, block, 0, (hipStream_t)stream, p);
-    return (int)hipGetLastError();
-}
-
 template <int D>
 static void launch_prep_d(const PrepParams &a, const PrepParams &b, int blocks_a, dim3 grid,
                           hipStream_t st) {
@@ -803,7 +804,8 @@ static void launch_prep_d(const PrepParams &a, const PrepParams &b, int blocks_a
 }
 
 static int prep_blocks(const PrepParams &p) {
-    return (int)(((int64_t)p.B * p.L + kPrepRows - 1) / kPrepRows);
+    const int rows = p.sumsq && !p.out ? NT : kPrepRows;   // of a workgroup
+    return (int)(((int64_t)p.B * p.L + rows - 1) / rows);
 }
 
 int launch_prep(const PrepParams &p, int D, void *stream) {

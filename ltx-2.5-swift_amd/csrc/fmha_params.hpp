@@ -75,7 +75,7 @@ struct PrepParams {
     float *rstd;                     // [B][L_full] or null
     void *out;                       // bf16 [B][L][H*D] contiguous or null
     // Statistic given as partial sums of squares (row b*L_full + l at sumsq + row*ss_rs,
-    // ss_blocks partials), or null: computed from x.
+    // ss_blocks partials), or null: computed from x. With it and no out, x is not read.
     const float *sumsq;
     int64_t ss_rs;
     int32_t ss_blocks;
@@ -130,16 +130,6 @@ struct LinearParams {
 
 // Tiles of linear_ks.hip, whose waves split the reduction: rows x columns of y.
 enum LinearKsTile { kLinearKs128 = 1, kLinearKs64 = 2, kLinearKs64x32 = 3, kLinearKs32 = 4 };
-
-// RMS statistic from partial sums of squares: rstd[row] = 1/sqrt(sum_j parts[row][j] / n + eps)
-// for rows [0, rows); parts row r at sumsq + r*rs, `blocks` partials.
-struct RstdParams {
-    const float *sumsq;
-    int64_t rs;
-    int32_t rows, blocks, n;
-    float eps;
-    float *rstd;
-};
 
 // Gemma-4 text-encoder attention (gemma_attn.hip). The prologue normalises (per head over D),
 // rotates and scales q and k into q' [B][Hq][T][D], k' [B][Hkv][T][D], and normalises v into
@@ -213,11 +203,10 @@ int launch_fmha_dma(const FmhaParams &p, int D, void *stream);   // fmha_dma.hip
 int launch_fmha_short(const FmhaParams &p, int D, void *stream); // fmha_short.hip
 int launch_fmha_splitk(const FmhaParams &p, int D, void *stream);  // fmha_splitk.hip
 int launch_prep(const PrepParams &p, int D, void *stream);
-// Two row sets in one launch (a call's Q statistic and its K prologue); same H * D.
+// Two row sets in one launch (a call's Q and K passes); same H * D.
 int launch_prep2(const PrepParams &a, const PrepParams &b, int D, void *stream);
 int launch_combine(const CombineParams &p, int D, void *stream);
 int launch_passthrough(const PassParams &p, int D, void *stream);
-int launch_rstd(const RstdParams &p, void *stream);
 int launch_linear(const LinearParams &p, void *stream);           // linear_gemm.hip
 // linear_ks.hip: every tile whole, in tiles of LinearKsTile; p.part (float [M][column tiles])
 // when p.sumsq is set and the call has more than one column tile. p.tiles_*, n_full, splits

@@ -573,34 +573,22 @@ ltx_attn_status ltx_attn_fwd(const ltx_attn_args *a, void *stream) {
         return LTX_ATTN_OK;
     }
 
-    // 1. prologue passes: statistics (and, for the K prologue, the prepared K). A call that
-    // takes both its Q statistic and its K pass from the inputs runs them as one launch.
+    // 1. prologue passes: statistics (and, for the K prologue, the prepared K), in one launch.
     ltx::PrepParams qpp{}, kpp{};
     bool q_pass = false, k_pass = false;
-    if (pl.q_stat) {
-        ltx::RstdParams rp{};
-        rp.sumsq = a->q_sumsq; rp.rs = a->q_sumsq_rs;
-        rp.rows = B * a->Lq; rp.blocks = a->sumsq_blocks; rp.n = H * D; rp.eps = a->norm_eps;
-        rp.rstd = (float *)(ws + pl.off_qrstd);
-        if (int e = ltx::launch_rstd(rp, stream))
-            return fail(LTX_ATTN_EHIP, "q statistic launch: %s", hipGetErrorString((hipError_t)e));
-    } else if (pl.q_norm) {
+    if (pl.q_norm) {
         qpp.x = a->q; qpp.bs = a->q_bs; qpp.rs = a->q_rs; qpp.hs = a->q_hs;
         qpp.B = B; qpp.L = a->Lq; qpp.H = H;
         qpp.w = a->q_norm_w; qpp.eps = a->norm_eps;
+        if (pl.q_stat) {
+            qpp.sumsq = a->q_sumsq; qpp.ss_rs = a->q_sumsq_rs; qpp.ss_blocks = a->sumsq_blocks;
+        }
         qpp.rstd = (float *)(ws + pl.off_qrstd);
         q_pass = true;
     }
     const void *kptr = a->k;
     int64_t k_bs = a->k_bs, k_rs = a->k_rs, k_hs = a->k_hs;
-    if (pl.k_fused && pl.k_stat) {
-        ltx::RstdParams rp{};
-        rp.sumsq = a->k_sumsq; rp.rs = a->k_sumsq_rs;
-        rp.rows = B * a->Lk; rp.blocks = a->sumsq_blocks; rp.n = H * D; rp.eps = a->norm_eps;
-        rp.rstd = (float *)(ws + pl.off_krstd);
-        if (int e = ltx::launch_rstd(rp, stream))
-            return fail(LTX_ATTN_EHIP, "k statistic launch: %s", hipGetErrorString((hipError_t)e));
-    } else if (pl.k_prologue || (pl.k_fused && pl.k_norm)) {
+    if (pl.k_prologue || (pl.k_fused && pl.k_norm)) {
         kpp.x = a->k; kpp.bs = a->k_bs; kpp.rs = a->k_rs; kpp.hs = a->k_hs;
         kpp.B = B; kpp.L = pl.k_prologue ? pl.kprep_rows : a->Lk; kpp.L_full = a->Lk; kpp.H = H;
         kpp.w = a->k_norm_w; kpp.eps = a->norm_eps;
