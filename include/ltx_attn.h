@@ -248,6 +248,12 @@ size_t ltx_linear_workspace_bytes(const ltx_linear_args *a);
  * are not applied here. */
 ltx_attn_status ltx_linear(const ltx_linear_args *a, void *stream);
 
+/* Run `count` projections, in order as far as any reads or writes what another writes: what
+ * ltx_linear does for each. Up to four small ones that share one workspace, none depending on
+ * another (a module's to_q, to_k, to_v and gate), run as one launch. Every argument is checked
+ * before anything is launched. */
+ltx_attn_status ltx_linear_group(const ltx_linear_args *a, int32_t count, void *stream);
+
 /* ----------------------------------------------------------------------------------------
  * RoPE table construction (host side, no GPU): the reference builds these once per forward
  * and hands them to every block (DiTForward.swift:680-738).

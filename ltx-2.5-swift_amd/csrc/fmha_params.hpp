@@ -128,6 +128,14 @@ struct LinearParams {
     int32_t grid;
 };
 
+// Projections of one launch (linear_ks.hip): workgroups [first[i], first[i + 1]) run projection i.
+constexpr int kLinearGroup = 4;
+struct LinearGroup {
+    LinearParams p[kLinearGroup];
+    int32_t n;
+    int32_t first[kLinearGroup + 1], stat_first[kLinearGroup + 1];
+};
+
 // Tiles of linear_ks.hip, whose waves split the reduction: rows x columns of y.
 enum LinearKsTile { kLinearKs128 = 1, kLinearKs64 = 2, kLinearKs64x32 = 3, kLinearKs32 = 4 };
 
@@ -208,10 +216,10 @@ int launch_prep2(const PrepParams &a, const PrepParams &b, int D, void *stream);
 int launch_combine(const CombineParams &p, int D, void *stream);
 int launch_passthrough(const PassParams &p, int D, void *stream);
 int launch_linear(const LinearParams &p, void *stream);           // linear_gemm.hip
-// linear_ks.hip: every tile whole, in tiles of LinearKsTile; p.part (float [M][column tiles])
-// when p.sumsq is set and the call has more than one column tile. p.tiles_*, n_full, splits
-// and grid are not read.
-int launch_linear_ks(const LinearParams &p, int tile, void *stream);
+// linear_ks.hip: n <= kLinearGroup projections, none reading what another writes, every tile whole,
+// in tiles of LinearKsTile; p[i].part (float [M][column tiles]) when p[i].sumsq is set and the
+// projection has more than one column tile. p[i].tiles_*, n_full, splits and grid are not read.
+int launch_linear_ks(const LinearParams *p, int n, int tile, void *stream);
 int64_t linear_part_bytes(int64_t tail_tiles, int splits);          // one range: 256 KiB
 int launch_gemma_prep(const GemmaPrepParams &p, int D, void *stream);   // gemma_attn.hip
 int launch_gemma_attn(const GemmaAttnParams &p, int D, void *stream);

@@ -53,10 +53,18 @@ struct KsTile {
     static_assert(BYTES <= 160 * 1024, "LDS of one workgroup");
 };
 
-template <int MB, int NB, int KG>
+// GROUP: several projections (one is spared the look-up, about 1 us of a call's start).
+template <int MB, int NB, int KG, bool GROUP>
 __global__ __attribute__((amdgpu_flat_work_group_size(256 * KG, 256 * KG),
                           amdgpu_waves_per_eu(KG, KG)))
-void linear_ks_kernel(const LinearParams p) {
+void linear_ks_kernel(const LinearGroup grp) {
+    int which = 0;
+    if constexpr (GROUP) {
+#pragma unroll
+        for (int i = 1; i < kLinearGroup; ++i) which += (int)blockIdx.x >= grp.first[i] ? 1 : 0;
+    }
+    const LinearParams &p = grp.p[which];
+    const int wg = GROUP ? (int)blockIdx.x - grp.first[which] : (int)blockIdx.x;
     using T = KsTile<MB, NB, KG>;
     constexpr int TM = T::TM, TN = T::TN, NS = T::NS, CPS = T::CPS, WAVES = T::WAVES;
     __shared__ __attribute__((aligned(16))) char smem[T::BYTES];
@@ -72,7 +80,7 @@ void linear_ks_kernel(const LinearParams p) {
     // order, so the workgroups of one XCD share their x and w rows in its L2.
     int tm, tn;
     {
-        const int t = xcd_major(blockIdx.x, gridDim.x);
+        const int t = xcd_major(wg, GROUP ? p.tiles_m * p.tiles_n : (int)gridDim.x);
         constexpr int GRP = 8;
         const int group = t / (GRP * p.tiles_n), first = group * GRP;
         const int rows = min(GRP, p.tiles_m - first), within = t - group * GRP * p.tiles_n;
@@ -257,8 +265,13 @@ void linear_ks_kernel(const LinearParams p) {
 
 // Sums of squares over 256 columns from those of the column tiles (`per` tiles each, added in
 // order). One thread per (row, block).
-__global__ __launch_bounds__(256) void linear_stat_kernel(const LinearParams p, int blocks, int per) {
-    const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+__global__ __launch_bounds__(256) void linear_stat_kernel(const LinearGroup grp, int per) {
+    int which = 0;
+#pragma unroll
+    for (int i = 1; i < kLinearGroup; ++i) which += (int)blockIdx.x >= grp.stat_first[i] ? 1 : 0;
+    const LinearParams &p = grp.p[which];
+    const int blocks = (p.N + 255) / 256;
+    const int64_t i = (int64_t)((int)blockIdx.x - grp.stat_first[which]) * 256 + threadIdx.x;
     if (i >= (int64_t)p.M * blocks) return;
     const int m = (int)(i / blocks), j = (int)(i % blocks);
     const float *src = p.part + (int64_t)m * p.tiles_n;
@@ -268,31 +281,41 @@ __global__ __launch_bounds__(256) void linear_stat_kernel(const LinearParams p, 
 }
 
 template <int MB, int NB, int KG>
-int launch_ks(LinearParams p, hipStream_t st) {
+int launch_ks(const LinearParams *p, int n, hipStream_t st) {
     using T = KsTile<MB, NB, KG>;
-    p.tiles_m = (p.M + T::TM - 1) / T::TM;
-    p.tiles_n = (p.N + T::TN - 1) / T::TN;
-    const int64_t grid = (int64_t)p.tiles_m * p.tiles_n;
-    if (grid > 0x7fffffff) return (int)hipErrorInvalidValue;
-    hipLaunchKernelGGL((linear_ks_kernel<MB, NB, KG>), dim3((unsigned)grid), dim3(256 * KG), 0, st, p);
-    if (p.sumsq && p.tiles_n > 1) {
-        const int blocks = (p.N + 255) / 256;
-        const int64_t n = (int64_t)p.M * blocks;
-        hipLaunchKernelGGL(linear_stat_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st,
-                           p, blocks, 256 / T::TN);
+    LinearGroup grp{};
+    grp.n = n;
+    int64_t grid = 0, stat = 0;
+    for (int i = 0; i < kLinearGroup; ++i) {
+        grp.first[i] = (int32_t)grid;
+        grp.stat_first[i] = (int32_t)stat;
+        if (i >= n) continue;                        // (past the grid: chosen by no workgroup)
+        LinearParams &q = grp.p[i] = p[i];
+        q.tiles_m = (q.M + T::TM - 1) / T::TM;
+        q.tiles_n = (q.N + T::TN - 1) / T::TN;
+        grid += (int64_t)q.tiles_m * q.tiles_n;
+        if (q.sumsq && q.tiles_n > 1) stat += ((int64_t)q.M * ((q.N + 255) / 256) + 255) / 256;
+        if (grid > 0x7fffffff || stat > 0x7fffffff) return (int)hipErrorInvalidValue;
     }
+    grp.first[kLinearGroup] = (int32_t)grid;
+    grp.stat_first[kLinearGroup] = (int32_t)stat;
+    const dim3 g((unsigned)grid), b(256 * KG);
+    if (n > 1) hipLaunchKernelGGL((linear_ks_kernel<MB, NB, KG, true>), g, b, 0, st, grp);
+    else hipLaunchKernelGGL((linear_ks_kernel<MB, NB, KG, false>), g, b, 0, st, grp);
+    if (stat > 0)
+        hipLaunchKernelGGL(linear_stat_kernel, dim3((unsigned)stat), dim3(256), 0, st, grp, 256 / T::TN);
     return (int)hipGetLastError();
 }
 
 }  // namespace
 
-int launch_linear_ks(const LinearParams &p, int tile, void *stream) {
+int launch_linear_ks(const LinearParams *p, int n, int tile, void *stream) {
     hipStream_t st = (hipStream_t)stream;
     switch (tile) {
-    case kLinearKs128: return launch_ks<4, 4, 1>(p, st);
-    case kLinearKs64: return launch_ks<2, 2, 2>(p, st);
-    case kLinearKs64x32: return launch_ks<2, 1, 2>(p, st);
-    case kLinearKs32: return launch_ks<1, 1, 2>(p, st);
+    case kLinearKs128: return launch_ks<4, 4, 1>(p, n, st);
+    case kLinearKs64: return launch_ks<2, 2, 2>(p, n, st);
+    case kLinearKs64x32: return launch_ks<2, 1, 2>(p, n, st);
+    case kLinearKs32: return launch_ks<1, 1, 2>(p, n, st);
     }
     return (int)hipErrorInvalidValue;
 }

@@ -96,22 +96,27 @@ public:
         const int32_t Mq = batch * x.tokens, Mk = batch * kv.tokens;
         void *scratch = ws + L.attn;
         const size_t sb = L.lin_bytes;
-        project(w_.to_v, kv.data, kv.row_stride, Mk, v, n, nullptr, scratch, sb, stream);
-        if (!allPerturbed) {
-            project(w_.to_q, x.data, x.row_stride, Mq, q, n, qs, scratch, sb, stream);
-            project(w_.to_k, kv.data, kv.row_stride, Mk, k, n, ks, scratch, sb, stream);
-        }
         const bool gated = w_.to_gate_logits.weight != nullptr;
+        ltx_linear_args in[4];
+        int32_t nin = 0;
+        in[nin++] = projection(w_.to_v, kv.data, kv.row_stride, Mk, v, n, nullptr, scratch, sb);
+        if (!allPerturbed) {
+            in[nin++] = projection(w_.to_q, x.data, x.row_stride, Mq, q, n, qs, scratch, sb);
+            in[nin++] = projection(w_.to_k, kv.data, kv.row_stride, Mk, k, n, ks, scratch, sb);
+        }
         if (gated)
-            project(w_.to_gate_logits, x.data, x.row_stride, Mq, gate, heads, nullptr, scratch,
-                    sb, stream);
+            in[nin++] = projection(w_.to_gate_logits, x.data, x.row_stride, Mq, gate, heads, nullptr,
+                                   scratch, sb);
+        DiTAttention::check(ltx_linear_group(in, nin, stream));
         const DiTAttention::Stream sq{allPerturbed ? nullptr : q, (int64_t)x.tokens * n, n, x.tokens};
         const DiTAttention::Stream sk{allPerturbed ? nullptr : k, (int64_t)kv.tokens * n, n, kv.tokens};
         const DiTAttention::Stream sv{v, (int64_t)kv.tokens * n, n, kv.tokens};
         core_(batch, n, sq, sk, sv, merged, (int64_t)x.tokens * n, n, variant, rotary, keyRotary,
               ws + L.attn, L.attn_bytes, stream, k_valid_len, gated ? gate : nullptr,
               allPerturbed, allPerturbed ? nullptr : qs, allPerturbed ? nullptr : ks, blocks);
-        project(w_.to_out, merged, n, Mq, out, w_.to_out.out, nullptr, scratch, sb, stream);
+        const ltx_linear_args to_out =
+            projection(w_.to_out, merged, n, Mq, out, w_.to_out.out, nullptr, scratch, sb);
+        DiTAttention::check(ltx_linear(&to_out, stream));
     }
 
     size_t workspaceBytes(int32_t batch, const Input &x, const Input *context, Variant variant,
@@ -178,9 +183,9 @@ private:
 
     // y [M, out] = x [M, in] . w^T (+ b), rows of x `x_rs` apart; `sumsq` optional partials;
     // `scratch` the split tail's partial tiles.
-    static void project(const Linear &l, const void *x, int64_t x_rs, int32_t M, void *y,
-                        int32_t y_rs, float *sumsq, void *scratch, size_t scratch_bytes,
-                        void *stream) {
+    static ltx_linear_args projection(const Linear &l, const void *x, int64_t x_rs, int32_t M,
+                                      void *y, int32_t y_rs, float *sumsq, void *scratch,
+                                      size_t scratch_bytes) {
         ltx_linear_args a{};
         a.M = M; a.N = l.out; a.K = l.in;
         a.x = x; a.w = l.weight; a.bias = l.bias; a.y = y;
@@ -189,7 +194,7 @@ private:
         a.sumsq_rs = ltx_linear_sumsq_blocks(l.out);
         a.workspace = scratch;
         a.workspace_bytes = scratch_bytes;
-        DiTAttention::check(ltx_linear(&a, stream));
+        return a;
     }
 
     Weights w_;

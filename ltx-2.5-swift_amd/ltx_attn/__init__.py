@@ -22,6 +22,7 @@ from __future__ import annotations
 
 import ctypes
 import enum
+import functools
 import math
 import os
 from dataclasses import dataclass
@@ -121,7 +122,8 @@ EXPORTED_SYMBOLS = (
     "ltx_attn_status_string", "ltx_attn_last_error", "ltx_attn_provenance",
     "ltx_attn_abi_version", "ltx_attn_args_size", "ltx_rope_frequency_grid", "ltx_rope_video_positions",
     "ltx_rope_audio_positions", "ltx_rope_tables", "ltx_rope_tables_device",
-    "ltx_linear", "ltx_linear_sumsq_blocks", "ltx_linear_workspace_bytes", "ltx_gemma_attn_workspace_bytes",
+    "ltx_linear", "ltx_linear_group", "ltx_linear_sumsq_blocks", "ltx_linear_workspace_bytes",
+    "ltx_gemma_attn_workspace_bytes",
     "ltx_gemma_attn_fwd", "ltx_gemma_rope_tables", "ltx_device_count", "ltx_device_query",
     "ltx_attn_fwd_static", "ltx_rope_reference_positions",
     "ltx_rope_video_positions_with_references",
@@ -236,6 +238,8 @@ def load_library(path: str = LIB_PATH) -> ctypes.CDLL:
     lib.ltx_rope_tables_device.restype = ctypes.c_int
     lib.ltx_linear.argtypes = [ctypes.POINTER(LinearArgs), ctypes.c_void_p]
     lib.ltx_linear.restype = ctypes.c_int
+    lib.ltx_linear_group.argtypes = [ctypes.POINTER(LinearArgs), ctypes.c_int32, ctypes.c_void_p]
+    lib.ltx_linear_group.restype = ctypes.c_int
     lib.ltx_linear_workspace_bytes.argtypes = [ctypes.POINTER(LinearArgs)]
     lib.ltx_linear_workspace_bytes.restype = ctypes.c_size_t
     lib.ltx_linear_sumsq_blocks.argtypes = [ctypes.c_int32]
@@ -351,7 +355,12 @@ def _strides_split(t):
 
 
 def _ptr(t):
-    return None if t is None else ctypes.c_void_p(t.data_ptr())
+    return None if t is None else t.data_ptr()
+
+
+@functools.lru_cache(maxsize=64)
+def _default_scale(D: int) -> float:
+    return float(np.float32(1.0 / math.sqrt(D)))
 
 
 def attention_fwd(q, k, v, *, heads: int, layout: str = "merged", q_norm_w=None,
@@ -431,7 +440,7 @@ def attention_fwd(q, k, v, *, heads: int, layout: str = "merged", q_norm_w=None,
         arr = (ctypes.c_int32 * B)(*[int(x) for x in k_valid_len])
         keep.append(arr)
         a.k_valid_len = ctypes.cast(arr, ctypes.POINTER(ctypes.c_int32))
-    a.scale = float(np.float32(1.0 / math.sqrt(D))) if scale is None else float(scale)
+    a.scale = _default_scale(D) if scale is None else float(scale)
     a.out = _ptr(out)
     a.o_bs, a.o_rs, a.o_hs = os_
     a.kprep = kprep
@@ -467,9 +476,10 @@ def attention_fwd(q, k, v, *, heads: int, layout: str = "merged", q_norm_w=None,
         _check(lib.ltx_attn_fwd_static(ctypes.byref(a), ctypes.c_void_p(stream)))
         return out
     need = lib.ltx_attn_workspace_bytes(ctypes.byref(a))
-    st = lib.ltx_attn_validate(ctypes.byref(a))
-    if st not in (OK, EWORKSPACE):
-        _check(st)
+    if not need:                       # no workspace, or arguments that are refused
+        st = lib.ltx_attn_validate(ctypes.byref(a))
+        if st not in (OK, EWORKSPACE):
+            _check(st)
     if need and (workspace is None or workspace.numel() * workspace.element_size() < need + 256):
         workspace = torch.empty(need + 256, dtype=torch.uint8, device=q.device)
     if workspace is not None:
@@ -491,6 +501,7 @@ def linear_sumsq_blocks(n: int) -> int:
     return load_library().ltx_linear_sumsq_blocks(n)
 
 
+@functools.lru_cache(maxsize=1024)     # (a pure host function of the sizes)
 def linear_workspace_bytes(M: int, N: int, K: int) -> int:
     """Device scratch ``ltx_linear`` uses to split the tiles past its last whole round along K
     (0 when it would not split them)."""
@@ -499,22 +510,10 @@ def linear_workspace_bytes(M: int, N: int, K: int) -> int:
     return load_library().ltx_linear_workspace_bytes(ctypes.byref(a))
 
 
-def linear(x, weight, bias=None, *, out=None, sumsq=False, stream=None, workspace=None,
-           resident_groups: int = 0):
-    """``linear(_:_:)`` of ``DiTAttention.swift:178-188`` through ``ltx_linear``:
-    ``y = x . weight^T (+ bias)``, bf16 in and out, fp32 accumulation.
-
-    ``x``: bf16 ``[..., K]`` with a unit last stride (leading axes are flattened to rows, so
-    they must be collapsible); ``weight``: bf16 ``[N, K]`` (the checkpoint's layout);
-    ``bias``: bf16 ``[N]`` or None. ``out``: optional bf16 ``[..., N]`` view to write (unit
-    last stride; e.g. a column slice of a fused buffer). ``sumsq=True`` also returns the
-    statistic partials: fp32 ``[rows, ceil(N/256)]``, partial j of a row being the sum of
-    squares of its bf16 outputs over columns ``[256 j, 256 j + 256)``. ``workspace``: a
-    device tensor of at least ``linear_workspace_bytes(M, N, K)`` bytes for the split tail;
-    None allocates one when the shape splits, ``False`` runs every tile whole.
-    ``resident_groups``: as in ``attention_fwd`` (0: the device's CU count).
-    Returns ``y`` or ``(y, partials)``.
-    """
+def _linear_args(a, x, weight, bias, out, sumsq, resident_groups=0):
+    """Check a projection's tensors and fill its arguments (all but the workspace); its output,
+    statistic partials (None without ``sumsq``) and input rows, which may be a copy that has to
+    live until the launch."""
     import torch
 
     lib = load_library()
@@ -536,7 +535,6 @@ def linear(x, weight, bias=None, *, out=None, sumsq=False, stream=None, workspac
     y2 = out.view(-1, N) if out.dim() != 2 else out
     if bias is not None and (bias.dim() != 1 or bias.shape[0] != N or not bias.is_contiguous()):
         raise Failure(EINVAL, f"bias must be a contiguous [{N}] tensor")
-    a = LinearArgs()
     a.M, a.N, a.K = M, N, K
     a.resident_groups = resident_groups
     a.x, a.w, a.bias, a.y = _ptr(x2), _ptr(weight), _ptr(bias), _ptr(y2)
@@ -545,12 +543,37 @@ def linear(x, weight, bias=None, *, out=None, sumsq=False, stream=None, workspac
     a.y_rs = y2.stride(0) if M > 1 else N
     parts = None
     if sumsq:
-        nb = lib.ltx_linear_sumsq_blocks(N)
+        nb = -(-N // 256)              # ltx_linear_sumsq_blocks
         parts = torch.empty((M, nb), dtype=torch.float32, device=x.device)
         a.sumsq, a.sumsq_rs = _ptr(parts), nb
-    need = lib.ltx_linear_workspace_bytes(ctypes.byref(a)) if M > 0 else 0
-    if workspace is None and need:
-        workspace = torch.empty(need, dtype=torch.uint8, device=x.device)
+    return out, parts, x2
+
+
+def linear(x, weight, bias=None, *, out=None, sumsq=False, stream=None, workspace=None,
+           resident_groups: int = 0):
+    """``linear(_:_:)`` of ``DiTAttention.swift:178-188`` through ``ltx_linear``:
+    ``y = x . weight^T (+ bias)``, bf16 in and out, fp32 accumulation.
+
+    ``x``: bf16 ``[..., K]`` with a unit last stride (leading axes are flattened to rows, so
+    they must be collapsible); ``weight``: bf16 ``[N, K]`` (the checkpoint's layout);
+    ``bias``: bf16 ``[N]`` or None. ``out``: optional bf16 ``[..., N]`` view to write (unit
+    last stride; e.g. a column slice of a fused buffer). ``sumsq=True`` also returns the
+    statistic partials: fp32 ``[rows, ceil(N/256)]``, partial j of a row being the sum of
+    squares of its bf16 outputs over columns ``[256 j, 256 j + 256)``. ``workspace``: a
+    device tensor of at least ``linear_workspace_bytes(M, N, K)`` bytes for the split tail;
+    None allocates one when the shape splits, ``False`` runs every tile whole.
+    ``resident_groups``: as in ``attention_fwd`` (0: the device's CU count).
+    Returns ``y`` or ``(y, partials)``.
+    """
+    import torch
+
+    lib = load_library()
+    a = LinearArgs()
+    out, parts, x2 = _linear_args(a, x, weight, bias, out, sumsq, resident_groups)
+    if workspace is None:
+        need = linear_workspace_bytes(a.M, a.N, a.K) if a.M > 0 else 0
+        if need:
+            workspace = torch.empty(need, dtype=torch.uint8, device=x.device)
     if workspace is not None and workspace is not False:
         nbytes = workspace.numel() * workspace.element_size()
         a.workspace, a.workspace_bytes = _ptr(workspace), nbytes
@@ -558,6 +581,27 @@ def linear(x, weight, bias=None, *, out=None, sumsq=False, stream=None, workspac
         stream = torch.cuda.current_stream(x.device).cuda_stream
     _check(lib.ltx_linear(ctypes.byref(a), ctypes.c_void_p(stream)))
     return (out, parts) if sumsq else out
+
+
+def linear_group(calls, *, workspace=None, stream=None):
+    """Several projections through ``ltx_linear_group``: one launch where they are small, do
+    not depend on one another and ``workspace`` holds each one's ``linear_workspace_bytes``; else
+    one after another. ``calls``: ``(x, weight, bias, sumsq)`` each, as in ``linear``.
+    Returns a ``(y, partials)`` each (partials None without sumsq).
+    """
+    import torch
+
+    lib = load_library()
+    args = (LinearArgs * len(calls))()
+    res = [_linear_args(a, x, w, b, None, sumsq) for a, (x, w, b, sumsq) in zip(args, calls)]
+    if workspace is not None:
+        nbytes, ptr = workspace.numel() * workspace.element_size(), workspace.data_ptr()
+        for a in args:
+            a.workspace, a.workspace_bytes = ptr, nbytes
+    if stream is None:
+        stream = torch.cuda.current_stream(calls[0][0].device).cuda_stream
+    _check(lib.ltx_linear_group(args, len(calls), ctypes.c_void_p(stream)))
+    return [(y, parts) for y, parts, _ in res]
 
 
 def workspace_bytes(**kw) -> int:
@@ -637,34 +681,56 @@ class DiTAttentionModule:
             raise Failure(EINVAL, f"to_q.weight {tuple(q.shape)} is not [k * {heads}, queryDim]")
         self.core = DiTAttentionCore(weights["q_norm.weight"], weights["k_norm.weight"], heads)
 
-    def _lin(self, t, name, sumsq=False, workspace=None):
+    def _lin(self, t, name, sumsq=False, workspace=None, stream=None):
         w = self.w[name + ".weight"]
         # the call's workspace doubles as the projection's split-tail scratch when it is
         # large enough (the projections and the attention run in stream order)
         need = linear_workspace_bytes(t.numel() // t.shape[-1], w.shape[0], w.shape[1])
         if workspace is not None and workspace.numel() * workspace.element_size() < need:
             workspace = None
-        return linear(t, w, self.w.get(name + ".bias"), sumsq=sumsq, workspace=workspace)
+        return linear(t, w, self.w.get(name + ".bias"), sumsq=sumsq, workspace=workspace,
+                      stream=stream)
+
+    def _lin_group(self, calls, workspace, stream):
+        """``(y, partials)`` of each ``(input, name, sumsq)``."""
+        need = max(linear_workspace_bytes(t.numel() // t.shape[-1], *self.w[n + ".weight"].shape)
+                   for t, n, _ in calls)
+        if workspace is None and need:
+            import torch
+
+            workspace = torch.empty(need, dtype=torch.uint8, device=calls[0][0].device)
+        if workspace is not None and workspace.numel() * workspace.element_size() < need:
+            return [r if sq else (r, None) for t, n, sq in calls
+                    for r in [self._lin(t, n, sumsq=sq, workspace=workspace, stream=stream)]]
+        return linear_group([(t, self.w[n + ".weight"], self.w.get(n + ".bias"), sq)
+                             for t, n, sq in calls], workspace=workspace, stream=stream)
 
     def __call__(self, x, context=None, *, variant: Variant, rotary: Optional[Rotary] = None,
                  key_rotary: Optional[Rotary] = None, k_valid_len=None,
                  all_perturbed: bool = False, workspace=None):
+        import torch
+
         kv = x if context is None else context                       # :327
         B, Lq, Lk = x.shape[0], x.shape[1], kv.shape[1]
-        v = self._lin(kv, "to_v", workspace=workspace)                # :341
-        gate = None
-        if "to_gate_logits.weight" in self.w:                          # :387-391
-            gate = self._lin(x, "to_gate_logits", workspace=workspace)
+        stream = torch.cuda.current_stream(x.device).cuda_stream
+        # to_v (:341), the gate's logits (:387-391), to_q and to_k with their statistic (:358-359)
+        calls = [(kv, "to_v", False)]
+        if "to_gate_logits.weight" in self.w:
+            calls.append((x, "to_gate_logits", False))
+        if not all_perturbed:
+            calls += [(x, "to_q", True), (kv, "to_k", True)]
+        res = self._lin_group(calls, workspace, stream)
+        v = res[0][0]
+        gate = res[1][0] if "to_gate_logits.weight" in self.w else None
         if all_perturbed:                                              # :351-356
             o = self.core(None, None, v, variant=variant, gate_logits=gate, all_perturbed=True,
-                          workspace=workspace)
+                          workspace=workspace, stream=stream)
         else:
-            q, qs = self._lin(x, "to_q", sumsq=True, workspace=workspace)     # :358-359
-            k, ks = self._lin(kv, "to_k", sumsq=True, workspace=workspace)
+            (q, qs), (k, ks) = res[-2:]
             o = self.core(q, k, v, variant=variant, rotary=rotary, key_rotary=key_rotary,
                           k_valid_len=k_valid_len, gate_logits=gate, workspace=workspace,
-                          q_sumsq=qs.view(B * Lq, -1), k_sumsq=ks.view(B * Lk, -1))
-        return self._lin(o, "to_out.0", workspace=workspace)          # :402-404
+                          q_sumsq=qs.view(B * Lq, -1), k_sumsq=ks.view(B * Lk, -1), stream=stream)
+        return self._lin(o, "to_out.0", workspace=workspace, stream=stream)   # :402-404
 
 
 class DiTBlockAttention:

@@ -374,3 +374,68 @@ def test_linear_random_shapes(device, i):
     check_linear(yb, x, w, b, f"random {i}")
     if parts is not None:
         check_partials(parts.cpu().numpy(), yb, f"random {i}")
+
+
+@pytest.mark.parametrize("rows", [1, 33, 126, 300])
+@pytest.mark.parametrize("shared_input", [True, False])
+def test_group_is_the_projections_one_by_one(device, rows, shared_input):
+    """``linear_group`` (one launch of up to four small projections, a tile for all of them)
+    against each projection by itself: the same products, in another order of summation. A bf16
+    result may round the other way, once before and once after the bias: at most two bf16 steps
+    (2 ** -8 relative each), of the row's magnitude where the sum cancels."""
+    import torch
+
+    g = torch.Generator(device=device).manual_seed(rows)
+
+    def rand(*shape, std=1.0):
+        return (torch.randn(shape, generator=g, device=device) * std).to(torch.bfloat16)
+
+    K = 2048
+    xs = [rand(rows, K)]
+    if not shared_input:
+        xs.append(rand(77, 1024))
+    calls = []
+    for i, (n, sumsq, bias) in enumerate([(2048, False, True), (32, False, True),
+                                          (2048, True, False), (1000, True, True)]):
+        x = xs[i % len(xs)]
+        calls.append((x, rand(n, x.shape[1], std=x.shape[1] ** -0.5),
+                      rand(n, std=0.1) if bias else None, sumsq))
+    ws = torch.empty(64 << 20, dtype=torch.uint8, device=device)
+    for _ in range(2):                               # again, over the first call's workspace
+        got = L.linear_group(calls, workspace=ws)
+        for (x, w, b, sumsq), (y, parts) in zip(calls, got):
+            ref = L.linear(x, w, b, sumsq=sumsq, workspace=ws)
+            ry, rp = ref if sumsq else (ref, None)
+            assert (y.float() - ry.float()).abs().max() <= 2 * 2 ** -8 * 4.0
+            truth = x.double() @ w.double().t() + (0 if b is None else b.double())
+            assert (y.double() - truth).norm() <= 1.05 * (ry.double() - truth).norm() + 1e-6
+            if sumsq:
+                pad = torch.zeros(y.shape[0], -y.shape[1] % 256, device=device)
+                mine = torch.cat([y.float().square(), pad], 1).view(y.shape[0], -1, 256).sum(-1)
+                assert torch.allclose(parts, mine, rtol=1e-5)
+            else:
+                assert parts is None
+
+
+def test_group_runs_dependent_projections_in_order(device):
+    """A projection that reads another's output runs after it."""
+    import torch
+
+    g = torch.Generator(device=device).manual_seed(5)
+    x = torch.randn((64, 256), generator=g, device=device).to(torch.bfloat16)
+    w = (torch.randn((256, 256), generator=g, device=device) / 16).to(torch.bfloat16)
+    ws = torch.empty(64 << 20, dtype=torch.uint8, device=device)
+    lib = L.load_library()
+    import ctypes
+
+    mid, out = torch.empty_like(x), torch.empty_like(x)
+    args = (L.LinearArgs * 2)()
+    for a, (i, o) in zip(args, ((x, mid), (mid, out))):
+        a.M, a.N, a.K = 64, 256, 256
+        a.x, a.w, a.y = i.data_ptr(), w.data_ptr(), o.data_ptr()
+        a.x_rs = a.w_rs = a.y_rs = 256
+        a.workspace, a.workspace_bytes = ws.data_ptr(), ws.numel()
+    assert lib.ltx_linear_group(args, 2, ctypes.c_void_p(
+        torch.cuda.current_stream().cuda_stream)) == L.OK
+    ref = L.linear(L.linear(x, w, workspace=ws), w, workspace=ws)
+    assert torch.equal(out, ref)
