@@ -7,6 +7,8 @@
 #include <math.h>
 #include <stdint.h>
 
+#include <type_traits>
+
 #include "fmha_params.hpp"
 
 namespace ltx {
@@ -107,7 +109,36 @@ __device__ __forceinline__ f32x16 splat16(float x) {
     return v;
 }
 
-__device__ __forceinline__ float xlane32(float x) { return __shfl_xor(x, 32, 64); }
+// The value of lane ^ 32, and of lane ^ 16: v_permlane32_swap / v_permlane16_swap with both
+// operands x leave one half's (even rows') values in every lane of the first result and the other's
+// in the second. VALU only: __shfl_xor takes them through LDS (ds_bpermute), a round trip of over
+// 100 cycles in the middle of a softmax step (with lane_sum below and 1 / sqrt for powf in the Gemma
+// prologue: 1024 tokens 43.2 -> 40.7 us a sliding and 92.6 -> 86.9 us a full call).
+__device__ __forceinline__ float xlane32(float x) {
+    const auto v = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+    return __uint_as_float(threadIdx.x & 32 ? v[0] : v[1]);
+}
+__device__ __forceinline__ float xlane16(float x) {
+    const auto v = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+    return __uint_as_float(threadIdx.x & 16 ? v[0] : v[1]);
+}
+
+// Sum over each run of N lanes (32 or 64), in every lane, by VALU exchanges: rotations within rows
+// of 16 (after a step the values repeat, so a rotation by n is the exchange with lane ^ n).
+template <int N>
+__device__ __forceinline__ float lane_sum(float x) {
+    auto ror = [](float v, auto n) __attribute__((always_inline)) {
+        return __uint_as_float(__builtin_amdgcn_update_dpp(
+            0u, __float_as_uint(v), 0x120 + decltype(n)::value, 0xf, 0xf, false));
+    };
+    x += ror(x, std::integral_constant<int, 8>{});
+    x += ror(x, std::integral_constant<int, 4>{});
+    x += ror(x, std::integral_constant<int, 2>{});
+    x += ror(x, std::integral_constant<int, 1>{});
+    x += xlane16(x);
+    if constexpr (N == 64) x += xlane32(x);
+    return x;
+}
 
 // Position of key k (0..63) inside a 64-key row of V^T: bits 2 and 3 swapped. A lane's B
 // operand of O^T = V^T.P^T holds keys {16h + 4g + 0..3, 16h + 8 + 4g + 0..3} of the S

@@ -614,8 +614,7 @@ __device__ __forceinline__ void qk_prep_rows(const PrepParams &p, int blk) {
                 for (int e = 0; e < 8; ++e) ss += a[e] * a[e] + c2[e] * c2[e];
             }
         }
-#pragma unroll
-        for (int off = 32; off >= 1; off >>= 1) ss += __shfl_xor(ss, off, 64);
+        ss = lane_sum<64>(ss);
         rstd = 1.0f / sqrtf(ss / (float)inner + p.eps);
         if (lane == 0 && p.rstd) p.rstd[frow] = rstd;
     }

@@ -4,7 +4,7 @@
 //
 // Three launches (the first is the whole prologue, its q/k rows and its v blocks side by side):
 //   gemma_prep_kernel   one wave per (batch row, token, head) row of q or k: the per-head
-//                       RMS norm (fp32, pow(mean + eps, -0.5), times the weight), rotate_half
+//                       RMS norm (fp32, (mean + eps)^-0.5, times the weight), rotate_half
 //                       RoPE with the fp32 tables, q scaled by scale*log2(e). Rounding points:
 //                       the reference's norm returns the input dtype (GemmaTextEncoder.swift
 //                       :114), so its normed q and k are bf16, and its fp32 RoPE leaves both
@@ -114,9 +114,8 @@ __device__ __forceinline__ void gemma_prep_rows(const GemmaPrepParams &p, int wg
         float ss = 0.f;
 #pragma unroll
         for (int e = 0; e < E; ++e) ss += x[e] * x[e];
-#pragma unroll
-        for (int off = LPR / 2; off >= 1; off >>= 1) ss += __shfl_xor(ss, off, 64);
-        const float rs = powf(ss / (float)D + p.eps, -0.5f);
+        ss = lane_sum<LPR>(ss);
+        const float rs = 1.0f / sqrtf(ss / (float)D + p.eps);
 #pragma unroll
         for (int e = 0; e < E; ++e) x[e] = (x[e] * rs) * (kind == 0 ? wq[e] : wk[e]);
         // rotate_half pairs channel c with c +- D/2: lane l holds channels E*l ..; its partner
@@ -125,7 +124,7 @@ __device__ __forceinline__ void gemma_prep_rows(const GemmaPrepParams &p, int wg
         float y[E];
 #pragma unroll
         for (int e = 0; e < E; ++e) {
-            const float other = __shfl_xor(x[e], LPR / 2, 64);
+            const float other = LPR == 64 ? xlane32(x[e]) : xlane16(x[e]);
             const float c = cs[j][e >> 2][e & 3], s = sn[j][e >> 2][e & 3];
             // first half: x1 c - x2 s; second half: x2 c + x1 s
             y[e] = (first ? x[e] * c - other * s : x[e] * c + other * s) * f;
@@ -187,9 +186,8 @@ __device__ __forceinline__ void gemma_vt_block(const GemmaPrepParams &p, int wg,
         float ss = 0.f;
 #pragma unroll
         for (int e = 0; e < E; ++e) ss += x[j][e] * x[j][e];
-#pragma unroll
-        for (int off = 32; off >= 1; off >>= 1) ss += __shfl_xor(ss, off, 64);
-        const float rs = powf(ss / (float)D + p.eps, -0.5f);
+        ss = lane_sum<64>(ss);
+        const float rs = 1.0f / sqrtf(ss / (float)D + p.eps);
 #pragma unroll
         for (int e = 0; e < E; ++e) tile[wave * RW + j][lane * E + e] = (_Float16)(x[j][e] * rs);
     }
