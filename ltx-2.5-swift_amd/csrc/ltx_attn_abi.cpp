@@ -419,13 +419,13 @@ int32_t gemma_chunk_blocks(int32_t T) {
 // whose partials fit in `rows`. A range spreads a long query block over several CUs at the price
 // of fp32 partials (written and read back at about 5 TB/s) and a merge launch; one workgroup runs
 // per CU, the longest ranges first. A block takes a workgroup 0.75 us at D 256 (two at a time) and
-// 1.9 us at D 512, its start and epilogue about 8 us. Measured at 1024 tokens, attention + merge,
-// one range / two / three: D 256 causal 36 / 27 + 7 / 25 + 9 us; D 512 over all keys 86 / 54 +
+// 2.1 us at D 512, its start and epilogue about 8 us. Measured at 1024 tokens, attention + merge,
+// one range / two / three: D 256 causal 36 / 27 + 7 / 25 + 9 us; D 512 over all keys 77 / 54 +
 // 16 / 77 + 21 us.
 int32_t gemma_run_chunk(const ltx_gemma_attn_args *a, int64_t rows) {
     const int nkb = (a->T + 31) / 32, qwg = ltx::gemma_queries_per_workgroup();
     const int least = (nkb + ltx::kGemmaMaxChunks - 1) / ltx::kGemmaMaxChunks;
-    const double block_us = a->D == 512 ? 1.9 : 0.75, start_us = 8.0, merge_us = 4.0;
+    const double block_us = a->D == 512 ? 2.1 : 0.75, start_us = 8.0, merge_us = 2.0;
     constexpr int kGroups = 256;
     const int step = std::max(2, (nkb / 16) & ~1);
     int32_t best = nkb;
