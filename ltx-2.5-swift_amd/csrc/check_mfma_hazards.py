@@ -17,6 +17,11 @@ register allocator and scheduler put things:
   * no result is still inside its window at a label or a branch (the padding never relies
     on one particular path).
 
+It also rejects a buffer load to LDS with a scalar offset. The range check of a raw buffer is on
+the per-lane offset; whether and how the scalar one enters it (added, subtracted from the length,
+left out) decides what a copy past the end or from an emptied resource reads. The kernels rely on
+such copies reading nothing, so their whole offset has to be the lane's.
+
 It also rejects any kernel of the file that spills to scratch memory (`.private_seg_size`
 above 0): the kernels are laid out to fit the register file, and a spill would otherwise
 only show as a slowdown.
@@ -114,6 +119,23 @@ def check(lines, name):
     return errors
 
 
+# buffer_load_<type> vOFF, s[RSRC], SOFF offen lds (the destination is M0's, so no data register)
+LDS_COPY = re.compile(r"buffer_load_\w+\s+(.*)\blds\b")
+
+
+def check_copies(lines, name):
+    errors = []
+    for no, raw in enumerate(lines, 1):
+        m = LDS_COPY.match(raw.strip().split(";")[0])
+        if not m:
+            continue
+        words = m.group(1).replace(",", " ").split()
+        if words[2] != "0" or "offen" not in words:
+            errors.append(f"{name}:{no}: `{raw.strip()}`: a copy to LDS with a scalar offset "
+                          f"(or without the lane's), outside the range check")
+    return errors
+
+
 def main(path, allow=()):
     """`allow`: (name substring, bytes) pairs -- a kernel whose symbol contains the substring
     may use up to that many bytes of scratch (a known, reviewed spill); any other spill, or a
@@ -128,7 +150,7 @@ def main(path, allow=()):
             fn = text[start].rstrip(":")
             body = text[start + 1:i + 1]
             count += sum(1 for l in body if re.match(r"\s*;\s*mfma_s\s", l))
-            errors += check(body, fn[:60])
+            errors += check(body, fn[:60]) + check_copies(body, fn[:60])
             start = None
     for m in re.finditer(r"\.set (\S+)\.private_seg_size, (\d+)", "\n".join(text)):
         limit = max([b for sub, b in allow if sub in m.group(1)], default=0)

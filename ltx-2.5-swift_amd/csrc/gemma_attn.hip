@@ -369,8 +369,8 @@ __device__ __forceinline__ void gemma_copy_q(const u32x4 &rq, char *area, int la
 #pragma unroll
     for (int j = 0; j < 8 * N; ++j) {
         const int row = 4 * j + (lane >> 4);
-        copy_at(rq, (uint32_t)(uintptr_t)(lds_void *)(area + j * 1024),
-                row * (D * 2) + 16 * ((lane & 15) ^ (row & 15)), col);
+        copy_plus(rq, (uint32_t)(uintptr_t)(lds_void *)(area + j * 1024),
+                  row * (D * 2) + 16 * ((lane & 15) ^ (row & 15)), col);
     }
 }
 __device__ __forceinline__ f16x8 gemma_q_opnd(const char *area, int row, int c, int g) {
@@ -470,9 +470,9 @@ void gemma_attn256_kernel(const GemmaAttnParams p) {
                 const int u = wave * COPIES + j;             // 1 KB unit of the block: K' then V'^T
                 const bool isk = u < KBYTES / 1024;
                 const int uu = isk ? u : u - KBYTES / 1024;
-                copy_at(isk ? rk : rv,
-                        (uint32_t)(uintptr_t)(lds_void *)(dst + k * BLOCK + u * 1024), lane * 16,
-                        kb * KBYTES + uu * 1024);
+                copy_plus(isk ? rk : rv,
+                          (uint32_t)(uintptr_t)(lds_void *)(dst + k * BLOCK + u * 1024), lane * 16,
+                          kb * KBYTES + uu * 1024);
             }
         }
     };
@@ -673,8 +673,8 @@ void gemma_attn512_kernel(const GemmaAttnParams p) {
     const u32x4 rv = rsrc_words((const _Float16 *)p.vt + head_off, (int64_t)nkb_all * KBYTES);
     auto copy1 = [&](const u32x4 &rs, char *stages, int i, int j) __attribute__((always_inline)) {
         const int u = wave * COPIES + j;
-        copy_at(rs, (uint32_t)(uintptr_t)(lds_void *)(stages + (i & 1) * KBYTES + u * 1024),
-                lane * 16, (kb_lo + i) * KBYTES + u * 1024);
+        copy_plus(rs, (uint32_t)(uintptr_t)(lds_void *)(stages + (i & 1) * KBYTES + u * 1024),
+                  lane * 16, (kb_lo + i) * KBYTES + u * 1024);
     };
     auto copy = [&](const u32x4 &rs, char *stages, int i) __attribute__((always_inline)) {
 #pragma unroll
@@ -931,8 +931,8 @@ void gemma_attn512_short_kernel(const GemmaAttnParams p) {
         for (int j = 0; j < COPIES; ++j) {
             const int u = wave * COPIES + j;         // 1 KB unit of the block: K' then V'^T
             const bool isk = wave < 2;
-            copy_at(isk ? rk : rv, (uint32_t)(uintptr_t)(lds_void *)(dst + u * 1024), lane * 16,
-                    (kb_lo + i) * KBYTES + (isk ? u : u - KBYTES / 1024) * 1024);
+            copy_plus(isk ? rk : rv, (uint32_t)(uintptr_t)(lds_void *)(dst + u * 1024), lane * 16,
+                      (kb_lo + i) * KBYTES + (isk ? u : u - KBYTES / 1024) * 1024);
         }
     };
     copy_block(0);

@@ -26,7 +26,10 @@ __device__ __forceinline__ void wait_copies_but() {
 // from the buffer at its offset to M0 + 16*lane. As one assembly statement the compiler sees
 // no memory load, so its waits never account for these; the kernel waits for them itself
 // (vmcnt). The s_nop is the wait state an M0 write needs before the load. The compiler keeps
-// nothing in M0 in these kernels, so the clobber costs nothing.
+// nothing in M0 in these kernels, so the clobber costs nothing. The whole offset is the lane's, the
+// scalar one 0: a lane whose offset is at or past the resource's length (all of them where the
+// length is 0) reads nothing and stores zeros, which a scalar offset outside that check would not
+// promise.
 __device__ __forceinline__ void copy_all(u32x4 rs, uint32_t lds_byte, int voff) {
     asm volatile(
         "s_mov_b32 m0, %0\n\t"
@@ -37,14 +40,16 @@ __device__ __forceinline__ void copy_all(u32x4 rs, uint32_t lds_byte, int voff) 
         : "m0", "memory");
 }
 
-// The same with part of the offset, `soff`, uniform.
-__device__ __forceinline__ void copy_at(u32x4 rs, uint32_t lds_byte, int voff, int soff) {
+// The same at `voff` plus a uniform `off`. The sum is formed here, in the place of the wait state,
+// so that no register holds it across a loop.
+__device__ __forceinline__ void copy_plus(u32x4 rs, uint32_t lds_byte, int voff, int off) {
+    int at;
     asm volatile(
-        "s_mov_b32 m0, %0\n\t"
-        "s_nop 0\n\t"
-        "buffer_load_dwordx4 %1, %2, %3 offen lds"
-        :
-        : "s"(lds_byte), "v"(voff), "s"(rs), "s"(soff)
+        "s_mov_b32 m0, %1\n\t"
+        "v_add_u32_e32 %0, %4, %2\n\t"
+        "buffer_load_dwordx4 %0, %3, 0 offen lds"
+        : "=&v"(at)
+        : "s"(lds_byte), "v"(voff), "s"(rs), "s"(off)
         : "m0", "memory");
 }
 

@@ -80,6 +80,27 @@ def test_built_kernel_passes():
     assert H.main(s) == 0
 
 
+def test_copy_with_a_scalar_offset_is_caught():
+    """A copy to LDS past the end reads nothing only by the range check of its lane's offset."""
+    ok = "\ts_mov_b32 m0, s4\n\ts_nop 0\n\tbuffer_load_dwordx4 v9, s[8:11], 0 offen lds\n"
+    assert H.check_copies(ok.split("\n"), "t") == []
+    assert H.check_copies(["\tbuffer_load_dwordx4 v[0:3], v9, s[8:11], s5 offen"], "t") == []
+    for bad in ("s5 offen", "0x400 offen", "0"):
+        text = ok.replace("0 offen", bad)
+        assert len(H.check_copies(text.split("\n"), "t")) == 1, bad
+
+
+@pytest.mark.parametrize("name", ["fmha_dma", "fmha_short", "fmha_splitk", "linear_gemm",
+                                  "linear_ks", "gemma_attn"])
+def test_built_copies_have_no_scalar_offset(name):
+    s = os.path.join(ROOT, "ltx-2.5-swift_amd", "_build", name + ".s")
+    if not os.path.exists(s):
+        pytest.skip("device assembly not built (make -C ltx-2.5-swift_amd/csrc)")
+    lines = open(s).read().split("\n")
+    assert any(H.LDS_COPY.match(l.strip()) for l in lines)
+    assert H.check_copies(lines, name) == []
+
+
 def test_scratch_spill_is_caught(tmp_path):
     text = ("_Zkernel:\n\ts_endpgm\n"
             "\t.set _Zkernel.private_seg_size, 316\n")
