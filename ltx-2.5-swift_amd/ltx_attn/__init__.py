@@ -712,7 +712,8 @@ class DiTAttentionModule:
 
         kv = x if context is None else context                       # :327
         B, Lq, Lk = x.shape[0], x.shape[1], kv.shape[1]
-        stream = torch.cuda.current_stream(x.device).cuda_stream
+        # (host tensors have no stream; the projections refuse them)
+        stream = torch.cuda.current_stream(x.device).cuda_stream if x.is_cuda else None
         # to_v (:341), the gate's logits (:387-391), to_q and to_k with their statistic (:358-359)
         calls = [(kv, "to_v", False)]
         if "to_gate_logits.weight" in self.w:

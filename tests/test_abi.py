@@ -612,3 +612,22 @@ def test_gemma_attention_rejects_bad_arguments():
     fv = (ctypes.c_int32 * 1)(1025)
     st, msg = status(args(first_valid=ctypes.cast(fv, ctypes.POINTER(ctypes.c_int32))))
     assert st == L.EINVAL and "first_valid" in msg
+
+
+@pytest.mark.parametrize("call", ["plain", "perturbed", "gated", "workspace", "float32"])
+def test_module_refuses_host_tensors(call):
+    """A module call with tensors that are not on a device is refused with the library's own
+    error, also where there is no device to ask for a stream."""
+    import torch
+
+    n = 256
+    w = {k + ".weight": torch.zeros(n, n, dtype=torch.bfloat16)
+         for k in ("to_q", "to_k", "to_v", "to_out.0")}
+    w["q_norm.weight"] = w["k_norm.weight"] = torch.ones(n, dtype=torch.bfloat16)
+    if call == "gated":
+        w["to_gate_logits.weight"] = torch.zeros(8, n, dtype=torch.bfloat16)
+    x = torch.zeros(1, 16, n, dtype=torch.float32 if call == "float32" else torch.bfloat16)
+    with pytest.raises(L.Failure, match="bf16 device tensor"):
+        L.DiTAttentionModule(w, 8)(
+            x, variant=L.Variant.audioSelf, all_perturbed=call == "perturbed",
+            workspace=torch.empty(1 << 20, dtype=torch.uint8) if call == "workspace" else None)
