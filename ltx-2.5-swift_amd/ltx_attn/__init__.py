@@ -24,6 +24,7 @@ import ctypes
 import enum
 import functools
 import math
+import operator
 import os
 from dataclasses import dataclass
 from typing import Optional, Sequence
@@ -502,12 +503,17 @@ def linear_sumsq_blocks(n: int) -> int:
 
 
 @functools.lru_cache(maxsize=1024)     # (a pure host function of the sizes)
-def linear_workspace_bytes(M: int, N: int, K: int) -> int:
-    """Device scratch ``ltx_linear`` uses to split the tiles past its last whole round along K
-    (0 when it would not split them)."""
+def _linear_workspace_bytes(M: int, N: int, K: int) -> int:
     a = LinearArgs()
     a.M, a.N, a.K = M, N, K
     return load_library().ltx_linear_workspace_bytes(ctypes.byref(a))
+
+
+def linear_workspace_bytes(M: int, N: int, K: int) -> int:
+    """Device scratch ``ltx_linear`` uses to split the tiles past its last whole round along K
+    (0 when it would not split them)."""
+    # plain ints only as keys: an equal float, or a tensor by its identity, would find another's
+    return _linear_workspace_bytes(operator.index(M), operator.index(N), operator.index(K))
 
 
 def _linear_args(a, x, weight, bias, out, sumsq, resident_groups=0):

@@ -631,3 +631,19 @@ def test_module_refuses_host_tensors(call):
         L.DiTAttentionModule(w, 8)(
             x, variant=L.Variant.audioSelf, all_perturbed=call == "perturbed",
             workspace=torch.empty(1 << 20, dtype=torch.uint8) if call == "workspace" else None)
+
+
+def test_linear_workspace_query_takes_whole_numbers_only():
+    """The query of a projection's workspace keeps its answers by size; whatever it has
+    answered before, a float stays refused and an object is asked for its value each time."""
+    import torch
+
+    need = L.linear_workspace_bytes(12480, 4096, 4096)
+    assert need > 0
+    with pytest.raises(TypeError):
+        L.linear_workspace_bytes(12480.0, 4096, 4096)
+    rows = torch.tensor(12480)
+    assert L.linear_workspace_bytes(rows, 4096, 4096) == need
+    rows.fill_(16384)                   # 1024 tiles: whole rounds, nothing to split
+    assert L.linear_workspace_bytes(rows, 4096, 4096) == 0
+    assert L.linear_workspace_bytes(M=np.int64(12480), N=4096, K=4096) == need
