@@ -188,6 +188,12 @@ def load_library(path: str = LIB_PATH) -> ctypes.CDLL:
                            "`python -c 'import __graft_entry__ as g; g.build()'` or "
                            "`make -C ltx-2.5-swift_amd/csrc`")
     lib = ctypes.CDLL(path)
+    missing = [s for s in EXPORTED_SYMBOLS if not hasattr(lib, s)]
+    if missing:
+        version = (f"ABI version {lib.ltx_attn_abi_version()}"
+                   if "ltx_attn_abi_version" not in missing else "no ABI version")
+        raise RuntimeError(f"{path} ({version}) has no {', '.join(missing)}: an older build than "
+                           "this binding; build it again (`make -C ltx-2.5-swift_amd/csrc`)")
     P = ctypes.POINTER(Args)
     lib.ltx_attn_args_init.argtypes = [P]
     lib.ltx_attn_args_init.restype = None

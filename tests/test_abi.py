@@ -647,3 +647,23 @@ def test_linear_workspace_query_takes_whole_numbers_only():
     rows.fill_(16384)                   # 1024 tiles: whole rounds, nothing to split
     assert L.linear_workspace_bytes(rows, 4096, 4096) == 0
     assert L.linear_workspace_bytes(M=np.int64(12480), N=4096, K=4096) == need
+
+
+@pytest.mark.parametrize("present", [(), ("ltx_attn_abi_version", "ltx_attn_args_size")])
+def test_library_without_a_symbol_is_refused_by_name(tmp_path, monkeypatch, present):
+    """A library built before a symbol was added fails to load with a message that names the
+    library, its version and what it lacks."""
+    src = "int ltx_attn_abi_version(void) { return 8; }\n" if present else "int other;\n"
+    if present:
+        src += f"unsigned long ltx_attn_args_size(void) {{ return {ctypes.sizeof(L.Args)}; }}\n"
+        src += "".join(f"void {s}(void) {{}}\n" for s in L.EXPORTED_SYMBOLS
+                       if s not in present + ("ltx_linear_group",))
+    (tmp_path / "old.c").write_text(src)
+    so = str(tmp_path / "old.so")
+    subprocess.run(["gcc", "-shared", "-fPIC", str(tmp_path / "old.c"), "-o", so], check=True)
+    monkeypatch.setattr(L, "_lib", None)
+    with pytest.raises(RuntimeError) as e:
+        L.load_library(so)
+    assert so in str(e.value) and "ltx_linear_group" in str(e.value)
+    assert ("version 8" in str(e.value)) == bool(present)
+    assert L._lib is None
