@@ -407,12 +407,15 @@ GemmaRanges gemma_ranges_of(const ltx_gemma_attn_args *a, int qwg, int chunk, in
     return g;
 }
 
-// The workspace a call asks for holds the partials of 64-query (D 512) or 128-query (D 256)
-// blocks in ranges of 16 key blocks (longer for prompts past 128 key blocks, so that a query
-// block never has more than the merge's kGemmaMaxChunks).
+// Prompts of more than kGemmaWhole key blocks may split. The least partials that a call's workspace
+// holds: those of 64-query (D 512) or 128-query (D 256) blocks in ranges of 16 key blocks (longer
+// for prompts past 128 key blocks, so that a query block never has more than the merge's
+// kGemmaMaxChunks).
+constexpr int kGemmaWhole = 16;
 int32_t gemma_chunk_blocks(int32_t T) {
     const int nkb = (T + 31) / 32;
-    return std::max(std::min(nkb, 16), (nkb + ltx::kGemmaMaxChunks - 1) / ltx::kGemmaMaxChunks);
+    return std::max(std::min(nkb, kGemmaWhole),
+                    (nkb + ltx::kGemmaMaxChunks - 1) / ltx::kGemmaMaxChunks);
 }
 
 // The range length a call runs with: the cheapest, by an estimate in us, of the even lengths
@@ -424,6 +427,7 @@ int32_t gemma_chunk_blocks(int32_t T) {
 // 16 / 77 + 21 us.
 int32_t gemma_run_chunk(const ltx_gemma_attn_args *a, int64_t rows) {
     const int nkb = (a->T + 31) / 32, qwg = ltx::gemma_queries_per_workgroup();
+    if (nkb <= kGemmaWhole) return nkb;
     const int least = (nkb + ltx::kGemmaMaxChunks - 1) / ltx::kGemmaMaxChunks;
     const double block_us = a->D == 512 ? 2.1 : 0.75, start_us = 8.0, merge_us = 2.0;
     constexpr int kGroups = 256;
@@ -446,7 +450,12 @@ int32_t gemma_run_chunk(const ltx_gemma_attn_args *a, int64_t rows) {
     return best;
 }
 
-ltx_attn_status gemma_plan(const ltx_gemma_attn_args *a, GemmaPlan *pl) {
+// `least`: the ranges and the size of a workspace that holds the least partials (above) and no more.
+// Else the ranges may take what 16-block ranges of the kernels' own blocks take, and the size
+// covers them: at D 512 those are 128 queries, and a padded prompt of 1024 tokens (930 of them
+// padding) needs 32768 rows where 64-query blocks need 30720, without which it ran one range on half
+// of the chip (86.9 us a call, with two ranges 78.2).
+ltx_attn_status gemma_plan(const ltx_gemma_attn_args *a, GemmaPlan *pl, bool least = false) {
     g_err[0] = 0;
     if (!a) return fail(LTX_ATTN_EINVAL, "args is NULL");
     if (a->B < 1 || a->T < 4 || a->Hq < 1 || a->Hkv < 1)
@@ -494,16 +503,17 @@ ltx_attn_status gemma_plan(const ltx_gemma_attn_args *a, GemmaPlan *pl) {
     pl->off_k = align_up(qn, 256);
     pl->off_v = pl->off_k + align_up(kn, 256);
     pl->bytes = pl->off_v + align_up(kn, 256);
-    const int64_t rows =
-        gemma_ranges_of(a, a->D == 512 ? 64 : 128, gemma_chunk_blocks(a->T), nullptr, nullptr).rows;
-    if ((a->T + 31) / 32 > gemma_chunk_blocks(a->T)) {
+    const int qwg = ltx::gemma_queries_per_workgroup();
+    const int32_t sized = gemma_chunk_blocks(a->T);
+    int64_t rows = gemma_ranges_of(a, a->D == 512 ? 64 : 128, sized, nullptr, nullptr).rows;
+    pl->chunk = gemma_run_chunk(
+        a, least ? rows : std::max(rows, gemma_ranges_of(a, qwg, sized, nullptr, nullptr).rows));
+    rows = std::max(rows, gemma_ranges_of(a, qwg, pl->chunk, pl->part_row0, pl->part_chunks).rows);
+    if (rows) {
         pl->off_po = pl->bytes;
         pl->off_pml = pl->off_po + align_up((size_t)rows * D * 4, 256);
         pl->bytes = pl->off_pml + align_up((size_t)rows * 2 * 4, 256);
     }
-    pl->chunk = gemma_run_chunk(a, rows);
-    gemma_ranges_of(a, ltx::gemma_queries_per_workgroup(), pl->chunk, pl->part_row0,
-                    pl->part_chunks);
     pl->nch_max = ((a->T + 31) / 32 + pl->chunk - 1) / pl->chunk;
     return LTX_ATTN_OK;
 }
@@ -714,6 +724,7 @@ size_t ltx_gemma_attn_workspace_bytes(const ltx_gemma_attn_args *a) {
 ltx_attn_status ltx_gemma_attn_fwd(const ltx_gemma_attn_args *a, void *stream) {
     GemmaPlan pl;
     if (ltx_attn_status s = gemma_plan(a, &pl)) return s;
+    if (a->workspace_bytes < pl.bytes) gemma_plan(a, &pl, true);
     if (!a->workspace || a->workspace_bytes < pl.bytes)
         return fail(LTX_ATTN_EWORKSPACE, "workspace of %zu bytes needed (got %zu at %p)",
                     pl.bytes, a->workspace_bytes, a->workspace);

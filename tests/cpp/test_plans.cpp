@@ -1,0 +1,163 @@
+// Plans and routes of the C ABI on the host: ltx_attn_abi.cpp compiled into this program with
+// launchers that record what they are given (nothing is launched, no HIP library is linked).
+//
+// Gemma: for a sweep of prompt lengths, head dims, windows, paddings and batches, every query
+// block's ranges cover its key blocks, at most kGemmaMaxChunks of them, and the partials they
+// write lie inside the workspace that the call asked for, apart from one another.
+#include <cstdio>
+#include <cstdint>
+#include <string>
+#include <vector>
+
+#include "../../ltx-2.5-swift_amd/csrc/ltx_attn_abi.cpp"
+
+static int failures = 0, checks = 0;
+static std::string where;
+#define EXPECT(cond)                                                                         \
+    do {                                                                                     \
+        ++checks;                                                                            \
+        if (!(cond) && ++failures <= 20)                                                     \
+            std::printf("FAIL line %d [%s]: %s\n", __LINE__, where.c_str(), #cond);          \
+    } while (0)
+
+// ---- the HIP runtime and the launchers ------------------------------------------------------
+static int g_cus = 256;                  // CUs of "the device"
+static ltx::GemmaAttnParams g_gemma;
+static int g_gemma_launches = 0;
+
+extern "C" {
+hipError_t hipGetDevice(int *d) { *d = 0; return hipSuccess; }
+hipError_t hipDeviceGetAttribute(int *v, hipDeviceAttribute_t, int) { *v = g_cus; return hipSuccess; }
+hipError_t hipGetLastError(void) { return hipSuccess; }
+const char *hipGetErrorString(hipError_t) { return ""; }
+hipError_t hipGetDeviceCount(int *n) { *n = 1; return hipSuccess; }
+hipError_t hipGetDeviceProperties(hipDeviceProp_t *, int) { return hipErrorInvalidDevice; }
+hipError_t hipEventRecord(hipEvent_t, hipStream_t) { return hipSuccess; }
+}
+namespace ltx {
+int launch_fmha(const FmhaParams &, int, int, void *) { return 0; }
+int launch_fmha_short(const FmhaParams &, int, void *) { return 0; }
+int launch_fmha_splitk(const FmhaParams &, int, void *) { return 0; }
+int launch_prep(const PrepParams &, int, void *) { return 0; }
+int launch_prep2(const PrepParams &, const PrepParams &, int, void *) { return 0; }
+int launch_combine(const CombineParams &, int, void *) { return 0; }
+int launch_passthrough(const PassParams &, int, void *) { return 0; }
+int launch_linear(const LinearParams &, void *) { return 0; }
+int launch_linear_ks(const LinearParams *, int, int, void *) { return 0; }
+int64_t linear_part_bytes(int64_t tiles, int splits) { return tiles * splits * (256 << 10); }
+int launch_gemma_prep(const GemmaPrepParams &, int, void *) { return 0; }
+int launch_gemma_attn(const GemmaAttnParams &p, int, void *) {
+    g_gemma = p;
+    ++g_gemma_launches;
+    return 0;
+}
+int gemma_queries_per_workgroup() { return 128; }
+}  // namespace ltx
+
+// A distinct address per buffer, never read.
+static void *fake(uintptr_t i) { return reinterpret_cast<void *>((uintptr_t)0x7f0000000000ull + (i << 36)); }
+
+// ---- Gemma ------------------------------------------------------------------------------------
+struct GemmaCall {
+    ltx_gemma_attn_args a{};
+    int32_t fv[ltx::kMaxBatch] = {};
+    GemmaCall(int B, int T, int D, int window, std::vector<int> first) {
+        a.B = B; a.T = T; a.D = D; a.Hq = 16; a.Hkv = D == 512 ? 1 : 8;
+        a.q = fake(1); a.k = fake(2); a.v = fake(3);
+        a.q_rs = (int64_t)a.Hq * D; a.k_rs = a.v_rs = (int64_t)a.Hkv * D;
+        a.q_bs = T * a.q_rs; a.k_bs = a.v_bs = T * a.k_rs;
+        a.q_norm_w = fake(4); a.k_norm_w = fake(5);
+        a.eps = 1e-6f; a.scale = 1.0f;
+        a.cos = (const float *)fake(6); a.sin = (const float *)fake(7);
+        a.window = window;
+        for (int b = 0; b < B; ++b) fv[b] = first[b];
+        a.first_valid = fv;
+        a.out = (float *)fake(8);
+        a.o_rs = a.q_rs; a.o_bs = a.q_bs;
+        a.workspace = fake(9);
+        where = "B" + std::to_string(B) + " T" + std::to_string(T) + " D" + std::to_string(D) +
+                " window " + std::to_string(window) + " first valid " + std::to_string(first[0]);
+    }
+};
+
+// The recorded launch against the arguments: ranges and partials.
+static void check_gemma_launch(const GemmaCall &c) {
+    const ltx::GemmaAttnParams &p = g_gemma;
+    const int qwg = 128, nkb = (c.a.T + 31) / 32;
+    EXPECT(p.chunk >= 1 && p.nch_max >= 1 && p.nch_max <= ltx::kGemmaMaxChunks);
+    EXPECT(p.chunk * p.nch_max >= nkb);
+    const char *end = (const char *)c.a.workspace + c.a.workspace_bytes;
+    int64_t row = 0;                         // where the batch rows' partials may start
+    for (int b = 0; b < c.a.B; ++b) {
+        int64_t ranges = 0;
+        for (int q0 = 0; q0 < c.a.T; q0 += qwg) {
+            const int len = ltx::gemma_key_hi(c.a.T, q0, qwg, c.fv[b]) -
+                            ltx::gemma_key_lo(q0, c.fv[b], c.a.window) + 1;
+            const int n = ltx::gemma_ranges(c.a.T, c.a.window, p.chunk, q0, qwg, c.fv[b]);
+            EXPECT(len >= 1 && n == (len + p.chunk - 1) / p.chunk && n <= p.nch_max);
+            if (n > 1) ranges += n;
+        }
+        EXPECT(p.part_chunks[b] == ranges);
+        EXPECT(p.part_row0[b] >= row);
+        row = p.part_row0[b] + c.a.Hq * ranges * qwg;
+        if (ranges) {
+            const char *o = (const char *)p.part_o, *ml = (const char *)p.part_ml;
+            EXPECT(o >= (const char *)p.vt + 2 * (size_t)c.a.B * c.a.Hkv * nkb * 32 * c.a.D);
+            EXPECT(o + row * c.a.D * 4 <= ml);
+            EXPECT(ml + row * 2 * 4 <= end);
+        }
+    }
+}
+
+// A prompt that fills its tokens with padding but for the last `real` runs as two ranges of half of
+// its key blocks, whatever their number: 16 heads x 8 query blocks are half of the CUs.
+static void test_gemma_padded_prompts_split() {
+    for (int real = 1; real <= 400; ++real) {
+        GemmaCall c(1, 1024, 512, 0, {1024 - real});
+        c.a.workspace_bytes = ltx_gemma_attn_workspace_bytes(&c.a);
+        EXPECT(ltx_gemma_attn_fwd(&c.a, nullptr) == LTX_ATTN_OK);
+        EXPECT(g_gemma.nch_max == 2 && g_gemma.chunk == 16);
+        // the size asked for before: accepted, with the ranges that it holds
+        const size_t before = 2 * 1024 * 512 * (16 + 1 + 1) +
+            (512 * 4 + 2 * 4) * (size_t)gemma_ranges_of(&c.a, 64, 16, nullptr, nullptr).rows;
+        EXPECT(before <= c.a.workspace_bytes);
+        c.a.workspace_bytes = before;
+        EXPECT(ltx_gemma_attn_fwd(&c.a, nullptr) == LTX_ATTN_OK);
+        check_gemma_launch(c);
+    }
+}
+
+template <class F>
+static void gemma_sweep(F each) {
+    std::vector<int> lengths;
+    for (int T = 4; T <= 1700; T += 4) lengths.push_back(T);
+    for (int T : {2044, 2048, 3000, 4096, 4160, 8192}) lengths.push_back(T);
+    for (int D : {256, 512})
+        for (int T : lengths)
+            for (int window : {0, 1, 17, 512, 1024})
+                for (int pad : {0, 1, T / 3, T - T / 8, T - 1, T}) {
+                    each(1, T, D, window, std::vector<int>{pad});
+                    if (T % 100 < 4) each(2, T, D, window, std::vector<int>{pad, T / 2});
+                }
+}
+
+static void test_gemma_partials_fit() {
+    gemma_sweep([](int B, int T, int D, int window, std::vector<int> pad) {
+        GemmaCall c(B, T, D, window, pad);
+        c.a.workspace_bytes = ltx_gemma_attn_workspace_bytes(&c.a);
+        EXPECT(c.a.workspace_bytes > 0);
+        EXPECT(ltx_gemma_attn_fwd(&c.a, nullptr) == LTX_ATTN_OK);
+        check_gemma_launch(c);
+        c.a.workspace_bytes -= 1;
+        const int before = g_gemma_launches;
+        if (ltx_gemma_attn_fwd(&c.a, nullptr) == LTX_ATTN_OK) check_gemma_launch(c);
+        else EXPECT(g_gemma_launches == before);
+    });
+}
+
+int main() {
+    test_gemma_partials_fit();
+    test_gemma_padded_prompts_split();
+    std::printf("%d checks, %d failure(s)\n", checks, failures);
+    return failures != 0;
+}

@@ -480,6 +480,18 @@ def test_cpp_host_mirror_error_behaviour(tmp_path):
     assert "0 failure(s)" in run.stdout
 
 
+def test_plans_and_routes_on_the_host(tmp_path):
+    """ltx_attn_abi.cpp compiled with launchers that record what they are given
+    (tests/cpp/test_plans.cpp): the Gemma key ranges and their partials over a sweep of prompts."""
+    src = os.path.join(ROOT, "tests", "cpp", "test_plans.cpp")
+    exe = str(tmp_path / "test_plans")
+    subprocess.run(["g++", "-std=c++17", "-O1", "-D__HIP_PLATFORM_AMD__", "-I/opt/rocm/include",
+                    src, "-o", exe], check=True, capture_output=True)
+    run = subprocess.run([exe], capture_output=True, text=True)
+    assert run.returncode == 0, run.stdout + run.stderr
+    assert " 0 failure(s)" in run.stdout
+
+
 def test_connector_rope_tables():
     """The embeddings connector's tables (EmbeddingsConnector.swift:218-248): positions
     arange(seq) over maxPos 4096, one positional dimension filling width/2 frequencies (no
