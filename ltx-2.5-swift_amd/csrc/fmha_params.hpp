@@ -195,6 +195,13 @@ constexpr int gemma_ranges(int T, int window, int chunk, int q0, int nq, int fv)
     return n;
 }
 
+// Prompts up to kGemmaShortTokens take 64 queries per workgroup at D = 512, in a kernel that knows no
+// key ranges (one workgroup per query block, the output written whole).
+constexpr int kGemmaShortTokens = 512;
+constexpr bool gemma_short(int D, int T, int nch_max) {
+    return D == 512 && T <= kGemmaShortTokens && nch_max == 1;
+}
+
 // Host side: set the calling thread's error detail (ltx_attn_last_error) from a printf
 // format and its va_list, and return `s`. Defined in ltx_attn_abi.cpp, not exported.
 __attribute__((visibility("hidden"))) int set_error_detail(int s, const char *fmt, va_list ap);

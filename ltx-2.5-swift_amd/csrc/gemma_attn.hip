@@ -236,9 +236,7 @@ __global__ __launch_bounds__(256) void gemma_prep_kernel(const GemmaPrepParams p
 // kNCW 16-channel chunks, V'^T and O in kNDW 32-channel blocks.
 constexpr int kGemmaQueries = 128;
 constexpr int kNCW = 256 / 16, kNDW = 256 / 32;
-// Prompts up to kGemmaShortTokens take 64 queries per workgroup at D = 512. They have one key range
-// (the host's plan splits only prompts of more than 16 key blocks).
-constexpr int kGemmaShortQueries = 64, kGemmaShortTokens = 512;
+constexpr int kGemmaShortQueries = 64;           // of the kernel for short prompts (gemma_short)
 
 // Key blocks of the query block [q0, q0 + nq): causal / window / padding bounds; a block with
 // rows inside the left padding (their rows have no allowed key) runs over all keys, those rows
@@ -1163,7 +1161,7 @@ int launch_gemma_attn(const GemmaAttnParams &p, int D, void *stream) {
     const int64_t per_layer = (int64_t)p.B * p.Hq * ((p.T + kGemmaQueries - 1) / kGemmaQueries);
     const dim3 grid((unsigned)(per_layer * p.nch_max));
     hipStream_t st = (hipStream_t)stream;
-    if (D == 512 && p.T <= kGemmaShortTokens)
+    if (gemma_short(D, p.T, p.nch_max))
         hipLaunchKernelGGL(gemma_attn512_short_kernel,
                            dim3((unsigned)((int64_t)p.B * p.Hq *
                                            ((p.T + kGemmaShortQueries - 1) / kGemmaShortQueries))),

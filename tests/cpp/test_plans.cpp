@@ -86,6 +86,15 @@ static void check_gemma_launch(const GemmaCall &c) {
     const int qwg = 128, nkb = (c.a.T + 31) / 32;
     EXPECT(p.chunk >= 1 && p.nch_max >= 1 && p.nch_max <= ltx::kGemmaMaxChunks);
     EXPECT(p.chunk * p.nch_max >= nkb);
+    // the kernel without key ranges only where no query block has a second one; a plan that splits
+    // a short prompt goes to the kernel that has them
+    EXPECT(!ltx::gemma_short(c.a.D, c.a.T, 2));
+    if (ltx::gemma_short(c.a.D, c.a.T, p.nch_max)) {
+        EXPECT(c.a.D == 512 && c.a.T <= 512);
+        for (int b = 0; b < c.a.B; ++b) EXPECT(p.part_chunks[b] == 0 && p.chunk >= nkb);
+    } else {
+        EXPECT(c.a.D != 512 || c.a.T > 512);
+    }
     const char *end = (const char *)c.a.workspace + c.a.workspace_bytes;
     int64_t row = 0;                         // where the batch rows' partials may start
     for (int b = 0; b < c.a.B; ++b) {
