@@ -34,9 +34,9 @@
 //                       and O^T += V^T.P^T with v' and P in fp16 (the reference's weights are
 //                       fp32; with the max fixed a weight stays below 2^kGemmaBound). A block
 //                       whose weights would pass 2^kGemmaBound sends the workgroup to an exact
-//                       pass over its range (D 256: online max with rescaling; D 512: the rows'
-//                       maxima first). O is written in fp32, the dtype the reference's explicit
-//                       path returns.
+//                       pass over its range (D 256: online max with rescaling; D 512: with the
+//                       maxima that the first pass saw). O is written in fp32, the dtype the
+//                       reference's explicit path returns.
 //   gemma_combine_kernel  the long query blocks' keys run as ranges (the host's plan) on
 //                       separate workgroups, each writing unnormalised O and (max, sum); the
 //                       merge rescales and adds them.
@@ -715,7 +715,7 @@ void gemma_attn512_kernel(const GemmaAttnParams p) {
 
     f32x16 o[NDW][2];
     float m, l;
-    bool overflow = false;                           // some row's weights passed the bound
+    float top = -INFINITY;                           // the largest S of this lane's keys
     f32x16 sc[2];                                    // partial S of the next step's block
     auto opnd = [&](const char *base, int unit) __attribute__((always_inline)) {
         return *(const __attribute__((address_space(3))) f16x8 *)(
@@ -753,7 +753,7 @@ void gemma_attn512_kernel(const GemmaAttnParams p) {
     };
 
     // A pass over the range's key blocks, each row's max fixed at its first block with an allowed
-    // key; when any row outgrows it, the rows' exact maxima, then a second pass with those.
+    // key; when any row outgrows it, a second pass with the rows' maxima, which the first has seen.
     m = -INFINITY;
     auto run = [&]() __attribute__((always_inline)) {
 #pragma unroll
@@ -799,8 +799,7 @@ void gemma_attn512_kernel(const GemmaAttnParams p) {
                         wh[e >> 3][(e >> 1) & 3] = pack_f16x2(ex[e], ex[e + 1]);
                     }
                 });
-                // (each lane holds half of the row's keys: either half's overflow counts)
-                overflow |= mx > m + kGemmaBound;
+                top = fmaxf(top, mx);
                 l += ts;
             } else {
                 copy(rkn, sK, i + 2);
@@ -808,7 +807,7 @@ void gemma_attn512_kernel(const GemmaAttnParams p) {
                 for (int e = 0; e < 16; ++e) s[e] += x[e >> 2][e & 3];
                 const float mx = gemma_mask_max(s, kb, k_lo, k_hi, g);
                 if (m == -INFINITY) m = mx;          // the row's first allowed keys
-                overflow |= mx > m + kGemmaBound;
+                top = fmaxf(top, mx);
                 l += gemma_weights(s, m, wh);
                 if (more) s_block(i + 1, [](int) {});
             }
@@ -839,26 +838,10 @@ void gemma_attn512_kernel(const GemmaAttnParams p) {
         wait_copies();
     };
     run();
-    if (__syncthreads_or(overflow)) {
-        m = -INFINITY;
-        for (int i = 0; i < nblk; ++i) {
-            __syncthreads();
-            copy(rk, sK, i);
-            wait_copies();
-            __syncthreads();
-            s_block(i, [](int) {});
-            pass_s();
-            __syncthreads();
-            f32x16 s = sc[0];
-#pragma unroll
-            for (int i4 = 0; i4 < 4; ++i4) {
-                const f32x4 x = *(const f32x4 *)(xsS + ((mate * 4 + i4) * 64 + lane) * 4);
-#pragma unroll
-                for (int e = 0; e < 4; ++e) s[4 * i4 + e] += x[e];
-            }
-            m = fmaxf(m, gemma_mask_max(s, kb_lo + i, k_lo, k_hi, g));
-        }
-        __syncthreads();
+    // (each lane holds half of the row's keys)
+    top = fmaxf(top, xlane32(top));
+    if (__syncthreads_or(top > m + kGemmaBound)) {
+        m = top;
         copy(rk, sK, 0);
         if (nblk > 1) copy(rk, sK, 1);
         copy(rv, sV, 0);
@@ -957,8 +940,8 @@ void gemma_attn512_short_kernel(const GemmaAttnParams p) {
 
     f32x16 o[NDW];
     float m = -INFINITY, l;
+    float top = -INFINITY;                           // the row's largest S
     const f32x16 zero = splat16(0.f);                // the S chains' first SrcC
-    bool overflow = false;                           // some row's weights passed the bound
     auto opnd = [&](const char *base, int unit) __attribute__((always_inline)) {
         return *(const __attribute__((address_space(3))) f16x8 *)(
             (lds_void *)(base + unit * 1024 + lane * 16));
@@ -1009,7 +992,7 @@ void gemma_attn512_short_kernel(const GemmaAttnParams p) {
             for (int db = 0; db < NDW; ++db) va0[db] = v_opnd(0, db);
             const float mx = gemma_mask_max(s, kb_lo + i, k_lo, k_hi, g);
             if (m == -INFINITY) m = mx;              // the row's first allowed keys
-            overflow |= mx > m + kGemmaBound;
+            top = fmaxf(top, mx);
             u32x4 wh[2];
             l += gemma_weights(s, m, wh);
 #pragma unroll
@@ -1024,14 +1007,8 @@ void gemma_attn512_short_kernel(const GemmaAttnParams p) {
         }
     };
     run();
-    if (__syncthreads_or(overflow)) {
-        m = -INFINITY;
-        copy_block(0);
-        for (int i = 0; i < nblk; ++i) {
-            f32x16 s = s_block(i);
-            m = fmaxf(m, gemma_mask_max(s, kb_lo + i, k_lo, k_hi, g));
-        }
-        __syncthreads();
+    if (__syncthreads_or(top > m + kGemmaBound)) {
+        m = top;
         copy_block(0);
         run();
     }

@@ -162,7 +162,9 @@ EDGES = {
     "full_T640": dict(T=640, kind="full", fv=[0]),
     "sliding_T92_large": dict(T=92, kind="sliding", fv=[0], wk_mean=3.0),
     "full_T132_large": dict(T=132, kind="full", fv=[0], wk_mean=3.0),
+    "full_T512_large": dict(T=512, kind="full", fv=[0], wk_mean=3.0),
     "full_T772_pad40_large": dict(T=772, kind="full", fv=[40], wk_mean=3.0),
+    "full_T1028_B2_large": dict(T=1028, kind="full", fv=[0, 900], wk_mean=3.0),
 }
 
 
