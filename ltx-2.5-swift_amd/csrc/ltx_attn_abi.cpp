@@ -418,28 +418,27 @@ int32_t gemma_chunk_blocks(int32_t T) {
                     (nkb + ltx::kGemmaMaxChunks - 1) / ltx::kGemmaMaxChunks);
 }
 
-// The range length a call runs with: the cheapest, by an estimate in us, of the even lengths
-// whose partials fit in `rows`. A range spreads a long query block over several CUs at the price
+// The range length a call runs with on a part of `cus` CUs: the cheapest, by an estimate in us, of
+// the even lengths whose partials fit in `rows`. A range spreads a long query block over several CUs at the price
 // of fp32 partials (written and read back at about 5 TB/s) and a merge launch; one workgroup runs
 // per CU, the longest ranges first. A block takes a workgroup 0.75 us at D 256 (two at a time) and
 // 2.1 us at D 512, its start and epilogue about 8 us. Measured at 1024 tokens, attention + merge,
 // one range / two / three: D 256 causal 36 / 27 + 7 / 25 + 9 us; D 512 over all keys 77 / 54 +
 // 16 / 77 + 21 us.
-int32_t gemma_run_chunk(const ltx_gemma_attn_args *a, int64_t rows) {
+int32_t gemma_run_chunk(const ltx_gemma_attn_args *a, int64_t rows, int64_t cus) {
     const int nkb = (a->T + 31) / 32, qwg = ltx::gemma_queries_per_workgroup();
     if (nkb <= kGemmaWhole) return nkb;
     const int least = (nkb + ltx::kGemmaMaxChunks - 1) / ltx::kGemmaMaxChunks;
     const double block_us = a->D == 512 ? 2.1 : 0.75, start_us = 8.0, merge_us = 2.0;
-    constexpr int kGroups = 256;
     const int step = std::max(2, (nkb / 16) & ~1);
     int32_t best = nkb;
     double best_us = 0.0;
     for (int c = nkb; c >= std::max(least, 4); c = (c - 1) / step * step) {
         const GemmaRanges g = gemma_ranges_of(a, qwg, c, nullptr, nullptr);
         if (g.rows > rows) continue;
-        const double avg = (g.blocks * block_us + g.groups * start_us) / kGroups;
+        const double avg = (g.blocks * block_us + g.groups * start_us) / (double)cus;
         const double us =
-            std::max(g.longest * block_us + start_us, avg + (g.groups > kGroups ? 0.25 : 0.0) *
+            std::max(g.longest * block_us + start_us, avg + (g.groups > cus ? 0.25 : 0.0) *
                                                                 g.longest * block_us) +
             (g.rows ? merge_us + (double)g.rows * a->D * 8 / 5e6 : 0.0);
         if (best_us == 0.0 || us < best_us) {
@@ -455,7 +454,8 @@ int32_t gemma_run_chunk(const ltx_gemma_attn_args *a, int64_t rows) {
 // covers them: at D 512 those are 128 queries, and a padded prompt of 1024 tokens (930 of them
 // padding) needs 32768 rows where 64-query blocks need 30720, without which it ran one range on half
 // of the chip (86.9 us a call, with two ranges 78.2).
-ltx_attn_status gemma_plan(const ltx_gemma_attn_args *a, GemmaPlan *pl, bool least = false) {
+ltx_attn_status gemma_plan(const ltx_gemma_attn_args *a, GemmaPlan *pl, bool least = false,
+                           int64_t cus = kConcurrentGroups) {
     g_err[0] = 0;
     if (!a) return fail(LTX_ATTN_EINVAL, "args is NULL");
     if (a->B < 1 || a->T < 4 || a->Hq < 1 || a->Hkv < 1)
@@ -507,7 +507,8 @@ ltx_attn_status gemma_plan(const ltx_gemma_attn_args *a, GemmaPlan *pl, bool lea
     const int32_t sized = gemma_chunk_blocks(a->T);
     int64_t rows = gemma_ranges_of(a, a->D == 512 ? 64 : 128, sized, nullptr, nullptr).rows;
     pl->chunk = gemma_run_chunk(
-        a, least ? rows : std::max(rows, gemma_ranges_of(a, qwg, sized, nullptr, nullptr).rows));
+        a, least ? rows : std::max(rows, gemma_ranges_of(a, qwg, sized, nullptr, nullptr).rows),
+        cus);
     rows = std::max(rows, gemma_ranges_of(a, qwg, pl->chunk, pl->part_row0, pl->part_chunks).rows);
     if (rows) {
         pl->off_po = pl->bytes;
@@ -724,6 +725,13 @@ size_t ltx_gemma_attn_workspace_bytes(const ltx_gemma_attn_args *a) {
 ltx_attn_status ltx_gemma_attn_fwd(const ltx_gemma_attn_args *a, void *stream) {
     GemmaPlan pl;
     if (ltx_attn_status s = gemma_plan(a, &pl)) return s;
+    // the device's own plan when the workspace covers it, else the one the size query returned, else
+    // the least
+    const int64_t cus = device_groups(0);
+    if (cus != kConcurrentGroups) {
+        GemmaPlan own;
+        if (!gemma_plan(a, &own, false, cus) && own.bytes <= a->workspace_bytes) pl = own;
+    }
     if (a->workspace_bytes < pl.bytes) gemma_plan(a, &pl, true);
     if (!a->workspace || a->workspace_bytes < pl.bytes)
         return fail(LTX_ATTN_EWORKSPACE, "workspace of %zu bytes needed (got %zu at %p)",

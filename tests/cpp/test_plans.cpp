@@ -118,6 +118,20 @@ static void check_gemma_launch(const GemmaCall &c) {
     }
 }
 
+template <class F>
+static void gemma_sweep(F each) {
+    std::vector<int> lengths;
+    for (int T = 4; T <= 1700; T += 4) lengths.push_back(T);
+    for (int T : {2044, 2048, 3000, 4096, 4160, 8192}) lengths.push_back(T);
+    for (int D : {256, 512})
+        for (int T : lengths)
+            for (int window : {0, 1, 17, 512, 1024})
+                for (int pad : {0, 1, T / 3, T - T / 8, T - 1, T}) {
+                    each(1, T, D, window, std::vector<int>{pad});
+                    if (T % 100 < 4) each(2, T, D, window, std::vector<int>{pad, T / 2});
+                }
+}
+
 // A prompt that fills its tokens with padding but for the last `real` runs as two ranges of half of
 // its key blocks, whatever their number: 16 heads x 8 query blocks are half of the CUs.
 static void test_gemma_padded_prompts_split() {
@@ -136,18 +150,29 @@ static void test_gemma_padded_prompts_split() {
     }
 }
 
-template <class F>
-static void gemma_sweep(F each) {
-    std::vector<int> lengths;
-    for (int T = 4; T <= 1700; T += 4) lengths.push_back(T);
-    for (int T : {2044, 2048, 3000, 4096, 4160, 8192}) lengths.push_back(T);
-    for (int D : {256, 512})
-        for (int T : lengths)
-            for (int window : {0, 1, 17, 512, 1024})
-                for (int pad : {0, 1, T / 3, T - T / 8, T - 1, T}) {
-                    each(1, T, D, window, std::vector<int>{pad});
-                    if (T % 100 < 4) each(2, T, D, window, std::vector<int>{pad, T / 2});
-                }
+// On a part with other CUs a call runs the ranges that suit them, where its workspace holds them.
+static void test_gemma_plan_for_other_parts() {
+    GemmaCall c(1, 1024, 512, 0, {0});       // 128 query blocks: half of 256 CUs, all of 128
+    c.a.workspace_bytes = ltx_gemma_attn_workspace_bytes(&c.a);
+    EXPECT(ltx_gemma_attn_fwd(&c.a, nullptr) == LTX_ATTN_OK && g_gemma.nch_max == 2);
+    const size_t need = c.a.workspace_bytes;
+    for (int cus : {32, 64, 80, 128, 304}) {
+        g_cus = cus;
+        g_device_cus[0] = 0;                 // (kept from the first query)
+        where = std::to_string(cus) + " CUs";
+        EXPECT(ltx_gemma_attn_workspace_bytes(&c.a) == need);
+        EXPECT(ltx_gemma_attn_fwd(&c.a, nullptr) == LTX_ATTN_OK);
+        EXPECT(g_gemma.nch_max == (cus < 128 ? 1 : 2));
+        check_gemma_launch(c);
+        gemma_sweep([](int B, int T, int D, int window, std::vector<int> pad) {
+            GemmaCall d(B, T, D, window, pad);
+            d.a.workspace_bytes = ltx_gemma_attn_workspace_bytes(&d.a);
+            EXPECT(ltx_gemma_attn_fwd(&d.a, nullptr) == LTX_ATTN_OK);
+            check_gemma_launch(d);
+        });
+    }
+    g_cus = 256;
+    g_device_cus[0] = 0;
 }
 
 static void test_gemma_partials_fit() {
@@ -167,6 +192,7 @@ static void test_gemma_partials_fit() {
 int main() {
     test_gemma_partials_fit();
     test_gemma_padded_prompts_split();
+    test_gemma_plan_for_other_parts();
     std::printf("%d checks, %d failure(s)\n", checks, failures);
     return failures != 0;
 }
