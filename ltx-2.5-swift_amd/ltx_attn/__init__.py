@@ -603,6 +603,8 @@ def linear_group(calls, *, workspace=None, stream=None):
     """
     import torch
 
+    if not calls:
+        return []
     lib = load_library()
     args = (LinearArgs * len(calls))()
     res = [_linear_args(a, x, w, b, None, sumsq) for a, (x, w, b, sumsq) in zip(args, calls)]

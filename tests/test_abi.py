@@ -645,6 +645,11 @@ def test_module_refuses_host_tensors(call):
             workspace=torch.empty(1 << 20, dtype=torch.uint8) if call == "workspace" else None)
 
 
+def test_empty_group_of_projections():
+    """No projections: no launch, no stream and no device needed (as ltx_linear_group's count 0)."""
+    assert L.linear_group([]) == []
+
+
 def test_linear_workspace_query_takes_whole_numbers_only():
     """The query of a projection's workspace keeps its answers by size; whatever it has
     answered before, a float stays refused and an object is asked for its value each time."""
