@@ -1005,7 +1005,9 @@ ltx_attn_status linear_prepare(const ltx_linear_args *a, LinearCall *call) {
             (a->sumsq && meet(wb, linear_span(a->sumsq, a->M, a->sumsq_rs, blocks, 4))))
             return fail(LTX_ATTN_EINVAL, "linear workspace overlaps x, w, y or sumsq");
         p.part = (float *)a->workspace;
-        // (the statistic's column sums take far less of the workspace than the ranges would)
+        // Only here, where the ranges' workspace is there, though the statistic's column sums take far
+        // less of it: a call without one asks for whole tiles (a tile's bits then depend on its own
+        // rows of x and w alone, so a fused projection equals the separate ones).
         if (ls.n_full == 0) {
             const LinearShape sh{a->M, a->N, a->K};
             call->ks = linear_ks_tile(&sh, 1, groups,

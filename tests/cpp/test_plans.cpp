@@ -4,6 +4,10 @@
 // Gemma: for a sweep of prompt lengths, head dims, windows, paddings and batches, every query
 // block's ranges cover its key blocks, at most kGemmaMaxChunks of them, and the partials they
 // write lie inside the workspace that the call asked for, apart from one another.
+//
+// Projections: which kernel a call takes, and the group call's contract: everything is checked
+// before anything is launched, at most kLinearGroup small independent projections of one workspace
+// in one launch, with their column sums apart inside it, everything else one by one in order.
 #include <cstdio>
 #include <cstdint>
 #include <string>
@@ -24,6 +28,11 @@ static std::string where;
 static int g_cus = 256;                  // CUs of "the device"
 static ltx::GemmaAttnParams g_gemma;
 static int g_gemma_launches = 0;
+struct LinearLaunch {
+    std::vector<ltx::LinearParams> p;    // one, or a group's
+    int tile;                            // of linear_ks.hip, or 0 for linear_gemm.hip
+};
+static std::vector<LinearLaunch> g_linear;
 
 extern "C" {
 hipError_t hipGetDevice(int *d) { *d = 0; return hipSuccess; }
@@ -42,8 +51,14 @@ int launch_prep(const PrepParams &, int, void *) { return 0; }
 int launch_prep2(const PrepParams &, const PrepParams &, int, void *) { return 0; }
 int launch_combine(const CombineParams &, int, void *) { return 0; }
 int launch_passthrough(const PassParams &, int, void *) { return 0; }
-int launch_linear(const LinearParams &, void *) { return 0; }
-int launch_linear_ks(const LinearParams *, int, int, void *) { return 0; }
+int launch_linear(const LinearParams &p, void *) {
+    g_linear.push_back({{p}, 0});
+    return 0;
+}
+int launch_linear_ks(const LinearParams *p, int n, int tile, void *) {
+    g_linear.push_back({std::vector<LinearParams>(p, p + n), tile});
+    return 0;
+}
 int64_t linear_part_bytes(int64_t tiles, int splits) { return tiles * splits * (256 << 10); }
 int launch_gemma_prep(const GemmaPrepParams &, int, void *) { return 0; }
 int launch_gemma_attn(const GemmaAttnParams &p, int, void *) {
@@ -189,10 +204,151 @@ static void test_gemma_partials_fit() {
     });
 }
 
+// ---- projections ------------------------------------------------------------------------------
+static ltx_linear_args linear(int id, int M, int N, int K, bool sumsq, size_t ws = 64 << 20) {
+    ltx_linear_args a{};
+    a.M = M; a.N = N; a.K = K;
+    a.x = fake(20 + 8 * id); a.w = fake(21 + 8 * id); a.bias = fake(22 + 8 * id); a.y = fake(23 + 8 * id);
+    a.x_rs = a.w_rs = K; a.y_rs = N;
+    if (sumsq) {
+        a.sumsq = (float *)fake(24 + 8 * id);
+        a.sumsq_rs = ltx_linear_sumsq_blocks(N);
+    }
+    a.workspace = ws ? fake(9) : nullptr;
+    a.workspace_bytes = ws;
+    return a;
+}
+
+// The route of a call: a tile of linear_ks.hip, or linear_gemm.hip's whole tiles, tail ranges behind
+// whole rounds, or ranges alone.
+enum Route { kWhole, kTail, kRanges, kKs };
+static Route route(const ltx_linear_args &a) {
+    g_linear.clear();
+    where = std::to_string(a.M) + " x " + std::to_string(a.N) + " x " + std::to_string(a.K);
+    EXPECT(ltx_linear(&a, nullptr) == LTX_ATTN_OK && g_linear.size() == 1);
+    const ltx::LinearParams &p = g_linear[0].p[0];
+    return g_linear[0].tile ? kKs : p.splits <= 1 ? kWhole : p.n_full > 0 ? kTail : kRanges;
+}
+
+static void test_linear_routes() {
+    auto at = [](int M, int N, int K, int groups = 0, size_t ws = 64 << 20) {
+        ltx_linear_args a = linear(0, M, N, K, true, ws);
+        a.resident_groups = groups;
+        return route(a);
+    };
+    // what the GPU tests of each route call (test_gpu_linear.py)
+    EXPECT(at(12480, 4096, 4096) == kTail);
+    EXPECT(at(3000, 1024, 512, 32) == kTail);
+    EXPECT(at(300, 12288, 4096) == kRanges);
+    EXPECT(at(512, 12288, 4096) == kRanges);
+    EXPECT(at(700, 1000, 4096, 150) == kRanges);
+    EXPECT(at(700, 6144, 4096) == kRanges);
+    for (auto s : {std::pair<int, int>{13, 2048}, {12480, 32}, {200, 4096}, {1024, 4096}})
+        EXPECT(at(s.first, s.second, 2048) == kKs);
+    EXPECT(at(3120, 4096, 4096) == kWhole);
+    EXPECT(at(12480, 32, 4096, 0, 0) == kWhole);          // no workspace: whole tiles
+    EXPECT(at(12480, 32, 4096, 0, 1 << 20) == kWhole);    // nor with less than the ranges' partials
+    // another part's plan where the workspace holds it
+    g_cus = 128;
+    g_device_cus[0] = 0;                     // (kept from the first query)
+    EXPECT(at(12480, 4096, 4096) == kTail && g_linear[0].p[0].n_full == 768);
+    g_cus = 256;
+    g_device_cus[0] = 0;
+}
+
+static void test_linear_group() {
+    using Calls = std::vector<ltx_linear_args>;
+    auto run = [](const Calls &c) {
+        g_linear.clear();
+        return ltx_linear_group(c.data(), (int32_t)c.size(), nullptr);
+    };
+    auto module = [](size_t ws = 64 << 20) {
+        return Calls{linear(0, 126, 2048, 2048, false, ws), linear(1, 126, 32, 2048, false, ws),
+                     linear(2, 126, 2048, 2048, true, ws), linear(3, 126, 2048, 2048, true, ws)};
+    };
+    where = "group";
+    EXPECT(ltx_linear_group(nullptr, 0, nullptr) == LTX_ATTN_OK);
+    EXPECT(ltx_linear_group(nullptr, 2, nullptr) == LTX_ATTN_EINVAL);
+    EXPECT(ltx_linear_group(nullptr, -1, nullptr) == LTX_ATTN_EINVAL);
+
+    // one launch, in the caller's order, the column sums apart and inside the workspace
+    Calls c = module();
+    EXPECT(run(c) == LTX_ATTN_OK && g_linear.size() == 1 && g_linear[0].p.size() == 4);
+    const char *ws = (const char *)c[0].workspace, *used = ws;
+    for (size_t i = 0; i < c.size() && i < g_linear[0].p.size(); ++i) {
+        const ltx::LinearParams &p = g_linear[0].p[i];
+        EXPECT(p.y == c[i].y && p.sumsq == c[i].sumsq);
+        if (!p.sumsq) continue;
+        EXPECT((const char *)p.part >= used && ((uintptr_t)p.part & 255) == 0);
+        used = (const char *)p.part + (size_t)p.M * ((p.N + 31) / 32) * 4;   // the narrowest tiles
+        EXPECT(used <= ws + c[i].workspace_bytes);
+    }
+    // a bad call in any place: nothing is launched
+    for (size_t bad = 0; bad < 6; ++bad) {
+        c = module();
+        c.push_back(linear(4, 40, 64, 256, false));
+        c.push_back(linear(5, 40, 64, 256, false));
+        c[bad].K = 96;
+        EXPECT(run(c) != LTX_ATTN_OK && g_linear.empty());
+    }
+    // one by one, in order: more than a launch takes, an empty or a large one among them, other
+    // workspaces
+    auto in_order = [&](const Calls &calls, size_t launches) {
+        EXPECT(run(calls) == LTX_ATTN_OK && g_linear.size() == launches);
+        size_t at = 0;
+        for (const LinearLaunch &l : g_linear) {
+            EXPECT(l.p.size() == 1);
+            while (at < calls.size() && calls[at].M == 0) ++at;
+            EXPECT(at < calls.size() && l.p[0].y == calls[at].y);
+            ++at;
+        }
+    };
+    c = module();
+    c.push_back(linear(4, 126, 2048, 2048, false));
+    in_order(c, 5);
+    c = module();
+    c[1].M = 0;
+    in_order(c, 3);
+    c = module();
+    c[0] = linear(0, 12480, 4096, 4096, false);
+    in_order(c, 4);
+    c = module();
+    c[3].workspace = fake(10);
+    in_order(c, 4);
+    c = module(0);
+    in_order(c, 4);
+    // less than a call's ranges would need: it keeps whole tiles, so the others run by themselves too.
+    // (A workspace that holds the ranges of each call, 8 bytes and more per element of its y, holds
+    // the column sums of four, an eighth of a byte each.)
+    c = module();
+    c[3].workspace_bytes = 1 << 20;
+    in_order(c, 4);
+    // one by one: a call that reads or writes what another one writes, its workspace included
+    auto apart = [&](auto change) {
+        Calls d = module();
+        change(d);
+        in_order(d, d.size());
+    };
+    apart([](Calls &d) { d[2].x = d[0].y; });
+    apart([](Calls &d) { d[0].x = d[2].y; });
+    apart([](Calls &d) { d[2].w = d[0].y; });
+    apart([](Calls &d) { d[1].bias = d[0].y; });
+    apart([](Calls &d) { d[3].y = (char *)d[2].y + 126 * 2048 * 2 - 8; });
+    apart([](Calls &d) { d[3].sumsq = d[2].sumsq; });
+    apart([](Calls &d) { d[3].sumsq = (float *)d[0].y; });
+    apart([](Calls &d) { d[3].bias = (char *)d[3].workspace + (1 << 20); });
+    // y slices interleaved in one buffer: their spans meet, so they run one by one
+    apart([](Calls &d) {
+        for (int i : {0, 2, 3}) { d[i].y = (char *)fake(23) + 4096 * i; d[i].y_rs = 4 * 2048; }
+    });
+}
+
 int main() {
     test_gemma_partials_fit();
     test_gemma_padded_prompts_split();
     test_gemma_plan_for_other_parts();
+    test_linear_routes();
+    test_linear_group();
     std::printf("%d checks, %d failure(s)\n", checks, failures);
     return failures != 0;
 }

@@ -482,7 +482,8 @@ def test_cpp_host_mirror_error_behaviour(tmp_path):
 
 def test_plans_and_routes_on_the_host(tmp_path):
     """ltx_attn_abi.cpp compiled with launchers that record what they are given
-    (tests/cpp/test_plans.cpp): the Gemma key ranges and their partials over a sweep of prompts."""
+    (tests/cpp/test_plans.cpp): the Gemma key ranges and their partials over a sweep of prompts,
+    the kernel each projection takes, and the group call's contract."""
     src = os.path.join(ROOT, "tests", "cpp", "test_plans.cpp")
     exe = str(tmp_path / "test_plans")
     subprocess.run(["g++", "-std=c++17", "-O1", "-D__HIP_PLATFORM_AMD__", "-I/opt/rocm/include",

@@ -119,8 +119,9 @@ def test_fused_projection_equals_separate_ones(device):
     """With every tile whole (no tail split), one GEMM over [to_q; to_k; to_v] weights writes
     the same bits, and the same statistic partials for the q and k column ranges (which start
     at multiples of 256), as three separate projections: each 256 x 256 tile depends only on
-    its own rows of x and w. With the tail split (36 and 12 tiles: 3 and 4 k ranges) the
-    summation order differs, so the two agree within the fp32 bound of check_linear."""
+    its own rows of x and w. With a workspace both take smaller tiles whose waves split the
+    reduction: the summation order differs, so the two agree within the fp32 bound of
+    check_linear."""
     import torch
 
     M, inner, K = 700, 1024, 2048
@@ -217,11 +218,13 @@ def test_attention_takes_the_projection_statistic(device, Lq, Lk):
 
 @pytest.mark.parametrize("M,N,K", [
     (12480, 4096, 4096),    # to_q at 12480 tokens: 784 tiles = 3 rounds + 16 tiles in 8 ranges
-    (12480, 32, 4096),      # to_gate_logits: 49 tiles in 4 ranges each
+    (12480, 32, 4096),      # to_gate_logits: 64 x 32 tiles whose waves split the reduction
+    (512, 12288, 4096),     # fused q/k/v of 512 rows: no whole round, 96 tiles in 2 ranges each
 ])
 def test_tail_split_matches_whole_tiles(device, M, N, K):
     """The tiles past the last whole round of 256, cut along K into ranges whose fp32 partials
-    the fixup kernel sums, against the same call with every tile whole (workspace=False):
+    the fixup kernel sums (or a call too small for that in smaller tiles), against the same call
+    with every tile whole (workspace=False):
     each element within twice the fp32 summation bound plus one bf16 step; rows of a whole
     tile and of the split tile row against the oracle; the statistic partials of every row."""
     import torch
@@ -258,8 +261,8 @@ def test_tail_split_matches_whole_tiles(device, M, N, K):
 def test_tail_split_for_other_part_sizes(device, groups):
     """ltx_linear splits its tail for the device's CU count (the resident_groups argument
     stands in for it) when the workspace sized for 256 CUs covers that split: 3000 x 1024 x 512 is 48
-    tiles; 32 groups split the 16 past one round two ways, 100 split all 48 two ways (as the
-    split sized for 256 does). The oracle on the rows of a whole tile and of a split one, and the
+    tiles; 32 groups split the 16 past one round two ways, 100 take the smaller tiles whose waves
+    split the reduction. The oracle on the rows of a whole tile and of a split one, and the
     statistic partials of every row."""
     import torch
 
@@ -278,6 +281,33 @@ def test_tail_split_for_other_part_sizes(device, groups):
     rows = np.r_[0:64, 1024:1088, M - 64:M]
     check_linear(yb[rows], np.ascontiguousarray(x[rows]), w, b, f"groups {groups} rows")
     check_partials(parts.cpu().numpy(), yb, f"groups {groups}")
+
+
+@pytest.mark.parametrize("M,N,K,groups,splits", [
+    (300, 12288, 4096, 0, 2),     # 96 tiles, ragged rows
+    (700, 6144, 4096, 0, 3),      # 72 tiles; the last range of K shorter than the others
+    (700, 1000, 4096, 150, 8),    # 12 tiles, ragged both ways, for a part of 150 CUs
+])
+def test_every_tile_in_ranges(device, M, N, K, groups, splits):
+    """Calls without a whole round of tiles that still take the k ranges: each tile's partials
+    merged by the fixup, with bias and statistic (tests/cpp/test_plans.cpp holds that these sizes
+    are not given to the smaller tiles). Rows of the first and last row tiles against the oracle."""
+    import torch
+
+    _say(f"linear all ranges M={M} N={N} K={K} groups={groups}")
+    x = O.randn_bf16_bits((M, K), 1700 + N)
+    w = O.randn_bf16_bits((N, K), 1800 + M, std=K ** -0.5)
+    b = O.randn_bf16_bits((N,), 1900 + M, std=0.5)
+    # one tile's partials per range at least: the call would not split with less
+    ws = torch.empty(((M + 255) // 256) * ((N + 255) // 256) * splits << 18, dtype=torch.uint8,
+                     device=device)
+    y, parts = L.linear(dev(x, device), dev(w, device), dev(b, device), sumsq=True, workspace=ws,
+                        resident_groups=groups)
+    torch.cuda.synchronize()
+    yb = host_bits(y)
+    rows = np.r_[0:24, M - 24:M]
+    check_linear(yb[rows], np.ascontiguousarray(x[rows]), w, b, f"{M}x{N}x{K} ranges")
+    check_partials(parts.cpu().numpy(), yb, f"{M}x{N}x{K} ranges")
 
 
 @pytest.mark.parametrize("K,groups", [(64, 3), (128, 8), (192, 3), (1024, 8)])
@@ -439,3 +469,37 @@ def test_group_runs_dependent_projections_in_order(device):
         torch.cuda.current_stream().cuda_stream)) == L.OK
     ref = L.linear(L.linear(x, w, workspace=ws), w, workspace=ws)
     assert torch.equal(out, ref)
+
+
+def test_group_of_five_with_an_empty_one_into_one_buffer(device):
+    """More projections than a launch takes, one of no rows, writing interleaved column slices of
+    one buffer: one after another, so each is bit for bit what ``linear`` gives."""
+    import ctypes
+
+    import torch
+
+    g = torch.Generator(device=device).manual_seed(6)
+    rows, K, widths = 90, 512, [256, 64, 512, 8, 264]
+    x = torch.randn((rows, K), generator=g, device=device).to(torch.bfloat16)
+    ws = [(torch.randn((n, K), generator=g, device=device) / 22).to(torch.bfloat16) for n in widths]
+    big = torch.full((rows, sum(widths) + 4), 3.0, dtype=torch.bfloat16, device=device)
+    scratch = torch.empty(64 << 20, dtype=torch.uint8, device=device)
+    args, at, out = (L.LinearArgs * 5)(), 0, []
+    for i, (a, w) in enumerate(zip(args, ws)):
+        y = big[:, at:at + widths[i]]
+        a.M, a.N, a.K = 0 if i == 1 else rows, widths[i], K
+        a.x, a.w, a.y = x.data_ptr(), w.data_ptr(), y.data_ptr()
+        a.x_rs = a.w_rs = K
+        a.y_rs = big.stride(0)
+        a.workspace, a.workspace_bytes = scratch.data_ptr(), scratch.numel()
+        at += widths[i]
+        out.append(y)
+    _say("linear group of five")
+    assert L.load_library().ltx_linear_group(args, 5, ctypes.c_void_p(
+        torch.cuda.current_stream().cuda_stream)) == L.OK
+    for i, (y, w) in enumerate(zip(out, ws)):
+        if i == 1:
+            assert torch.all(y == 3.0)
+        else:
+            assert torch.equal(y, L.linear(x, w, workspace=scratch)), i
+    assert torch.all(big[:, at:] == 3.0)
