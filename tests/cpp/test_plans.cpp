@@ -165,6 +165,24 @@ static void test_gemma_padded_prompts_split() {
     }
 }
 
+// The calls of the GPU tests that mean to merge ranges (test_gpu_gemma.py) do.
+static void test_gemma_ranges_of_few_heads() {
+    struct Case { int B, T, D, window, Hq; std::vector<int> pad; int ranges; };
+    for (const Case &k : {Case{2, 2052, 512, 0, 2, {1026, 100}, 5}, Case{1, 2052, 512, 0, 2, {0}, 5},
+                          Case{2, 3076, 256, 1500, 1, {1538, 100}, 6},
+                          Case{1, 8324, 256, 3000, 1, {100}, 6}}) {
+        GemmaCall c(k.B, k.T, k.D, k.window, k.pad);
+        c.a.Hq = k.Hq; c.a.Hkv = 1;
+        c.a.q_rs = c.a.o_rs = k.Hq * k.D; c.a.k_rs = c.a.v_rs = k.D;
+        c.a.q_bs = c.a.o_bs = k.T * c.a.q_rs; c.a.k_bs = c.a.v_bs = k.T * c.a.k_rs;
+        c.a.workspace_bytes = ltx_gemma_attn_workspace_bytes(&c.a);
+        EXPECT(c.a.workspace_bytes <= (size_t)256 << 20);
+        EXPECT(ltx_gemma_attn_fwd(&c.a, nullptr) == LTX_ATTN_OK && g_gemma.nch_max == k.ranges);
+        EXPECT(k.B == 1 || g_gemma.part_chunks[0] != g_gemma.part_chunks[1]);
+        check_gemma_launch(c);
+    }
+}
+
 // On a part with other CUs a call runs the ranges that suit them, where its workspace holds them.
 static void test_gemma_plan_for_other_parts() {
     GemmaCall c(1, 1024, 512, 0, {0});       // 128 query blocks: half of 256 CUs, all of 128
@@ -346,6 +364,7 @@ static void test_linear_group() {
 int main() {
     test_gemma_partials_fit();
     test_gemma_padded_prompts_split();
+    test_gemma_ranges_of_few_heads();
     test_gemma_plan_for_other_parts();
     test_linear_routes();
     test_linear_group();

@@ -175,8 +175,8 @@ def test_attention_takes_the_projection_statistic(device, Lq, Lk):
     """q and k from ltx_linear with their partials: the attention with q_sumsq / k_sumsq (no
     statistic pass over q and k) meets the tolerance against the oracle of the whole chain and
     agrees with the attention that computes the statistic itself. 700 queries take the LDS-DMA
-    kernel (the K prologue reads the partials), 200 the register kernel (the statistic kernel
-    feeds its fused K norm); 600 x 152 is a cross-modal shape with its own key tables."""
+    kernel (the K prologue reads the partials), 200 the register kernel (the prologue's
+    sums feed its fused K norm); 600 x 152 is a cross-modal shape with its own key tables."""
     import torch
 
     H, D, K = 16, 128, 1024
