@@ -429,8 +429,10 @@ __device__ __forceinline__ GemmaRows gemma_rows(const GemmaAttnParams &p, const 
 // two stages while the other is read; one barrier per step. Two waves per SIMD overlap: alone, a
 // wave's chain S -> softmax -> P.V leaves the matrix cores idle most of the time (four waves of
 // up to 512 registers took 1.8 us per 128 queries and key block, these 0.73 us, 1.46 us a step
-// against 1.0 us of products per SIMD). What bounds a step is LDS: 256 KB of operand reads and
-// 64 KB of copies. (Two sets of waves in opposite phases, one forming S while the other ran
+// against 1.0 us of products per SIMD). No unit is full: over 2 x 2048 causal tokens (87 us) the
+// matrix cores are busy 32% of the time, LDS (256 KB of operand reads and 64 KB of copies a step)
+// 20%, the address unit's queue is full 14%; waves wait for data or the barrier 32% and to issue 37%
+// of theirs, with two of them per SIMD to cover it. (Two sets of waves in opposite phases, one forming S while the other ran
 // softmax and P.V, with two barriers a step, measured 0.88 us.)
 __global__ __attribute__((amdgpu_flat_work_group_size(512, 512), amdgpu_waves_per_eu(2, 2)))
 void gemma_attn256_kernel(const GemmaAttnParams p) {
@@ -636,9 +638,10 @@ void gemma_attn256_kernel(const GemmaAttnParams p) {
 
 // D = 512: four waves (one per SIMD, up to 512 registers); a wave owns 64 queries over half of
 // the head, its mate the other half, so that each LDS operand read feeds two products (eight
-// waves of 32 queries x 256 channels read 256 KB per key block, which bound them: calls of 2 x
-// 1224 and 2 x 1472 causal tokens took 120 and 138 us, with this kernel 109 and 129; with 64
-// queries per workgroup 186 and 241). The mates split the softmax: each
+// waves of 32 queries x 256 channels read 256 KB per key block: calls of 2 x 1224 and 2 x 1472
+// causal tokens took 120 and 138 us where this kernel took 109 and 129; it now takes 103 and 125,
+// the kernel with 64 queries per workgroup 185 and 241; at 2 x 2048 the matrix cores are busy 41% of
+// 163 us). The mates split the softmax: each
 // completes S and forms P for 32 of the 64 queries, its own (local group 0; the mate's are group
 // 1), so a step passes S partials one way and P the other. Software pipeline: step i issues the
 // 32 products of S(i + 1) one at a time with a slice of the softmax of S(i) after each, then
@@ -886,8 +889,9 @@ void gemma_attn512_kernel(const GemmaAttnParams p) {
 // D = 512, short prompts: 64 queries per workgroup, a wave 32 of them over half of the head (its
 // partner wave the other half), one key block at a time, no key ranges. Twice as many
 // workgroups, each with half of the 128-query kernel's start and epilogue, which bound a prompt of
-// a few blocks: 72 / 144 / 256 / 512 tokens 23.4 / 26.1 / 33.9 / 53.2 us a call against 26.9 /
-// 28.8 / 37.5 / 54.7. From 544 tokens on (a split plan's first) the other kernel is the faster.
+// a few blocks: 72 / 144 / 256 / 384 / 512 tokens 18.5 / 22.4 / 31.7 / 40.2 / 49.9 us a call against
+// 23.0 / 25.7 / 35.2 / 42.5 / 51.4. Past 512 tokens a plan may have key ranges, which only the other
+// kernel has.
 __global__ __attribute__((amdgpu_flat_work_group_size(256, 256), amdgpu_waves_per_eu(1, 1)))
 void gemma_attn512_short_kernel(const GemmaAttnParams p) {
     constexpr int D = 512, QWG = kGemmaShortQueries, NCW = kNCW, NDW = kNDW;

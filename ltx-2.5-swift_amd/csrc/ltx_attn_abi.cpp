@@ -419,12 +419,14 @@ int32_t gemma_chunk_blocks(int32_t T) {
 }
 
 // The range length a call runs with on a part of `cus` CUs: the cheapest, by an estimate in us, of
-// the even lengths whose partials fit in `rows`. A range spreads a long query block over several CUs at the price
-// of fp32 partials (written and read back at about 5 TB/s) and a merge launch; one workgroup runs
-// per CU, the longest ranges first. A block takes a workgroup 0.75 us at D 256 (two at a time) and
-// 2.1 us at D 512, its start and epilogue about 8 us. Measured at 1024 tokens, attention + merge,
-// one range / two / three: D 256 causal 36 / 27 + 7 / 25 + 9 us; D 512 over all keys 77 / 54 +
-// 16 / 77 + 21 us.
+// the even lengths whose partials fit in `rows`. A range spreads a long query block over several CUs
+// at the price of fp32 partials (written and read back at about 5 TB/s) and a merge launch; one
+// workgroup runs per CU, the longest ranges first. A block takes a workgroup 0.75 us at D 256 (two at
+// a time) and 2.1 us at D 512, its start and epilogue about 8 us. Measured at 1024 tokens, attention +
+// merge, one range / two / three: D 256 causal 36 / 24 + 7 / 25 + 9 us; D 512 over all keys 77 /
+// 51 + 17 / 77 + 21 us. Ranges shorter than the workspace's (D 512, one prompt, 8 blocks each) would
+// take 544 to 768 tokens from 51 .. 58 to 47 .. 52 us a call, but 832 and 896 from 60 to 64 and 69,
+// where this estimate still prefers them.
 int32_t gemma_run_chunk(const ltx_gemma_attn_args *a, int64_t rows, int64_t cus) {
     const int nkb = (a->T + 31) / 32, qwg = ltx::gemma_queries_per_workgroup();
     if (nkb <= kGemmaWhole) return nkb;

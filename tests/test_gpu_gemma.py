@@ -101,9 +101,9 @@ CASES = {
     "full_T4160": dict(B=1, T=4160, kind="full", fv=[0], seed=0x5EED + 560, absolute_only=True),
     # k_norm weights 25x the checkpoint's: logits with a spread of ~70 (log2 units), so later
     # key blocks pass a row's first-block max by more than 2^15 and the workgroups rerun their
-    # range exactly (online maxima, or those that the first pass saw). Logits that large amplify the inputs' bf16
-    # rounding (the reference's own arithmetic is ~2e-2 off), so only the bound relative to
-    # the reference's arithmetic applies.
+    # range exactly (online maxima, or those that the first pass saw). Logits that large amplify
+    # the inputs' bf16 rounding (the reference's own arithmetic is ~2e-2 off), so only the bound
+    # relative to the reference's arithmetic applies.
     "sliding_1024_large_logits": dict(B=1, T=1024, kind="sliding", fv=[0], wk_mean=3.0,
                                       seed=0x5EED + 530, relative_only=True),
     "full_1024_large_logits": dict(B=1, T=1024, kind="full", fv=[0], wk_mean=3.0,
