@@ -429,7 +429,7 @@ __device__ __forceinline__ GemmaRows gemma_rows(const GemmaAttnParams &p, const 
 // two stages while the other is read; one barrier per step. Two waves per SIMD overlap: alone, a
 // wave's chain S -> softmax -> P.V leaves the matrix cores idle most of the time (four waves of
 // up to 512 registers took 1.8 us per 128 queries and key block, these 0.73 us, 1.46 us a step
-// against 1.0 us of products per SIMD). No unit is full: over 2 x 2048 causal tokens (87 us) the
+// against 1.0 us of products per SIMD). No unit is full: over 2 x 2048 tokens, window 1024 (87 us) the
 // matrix cores are busy 32% of the time, LDS (256 KB of operand reads and 64 KB of copies a step)
 // 20%, the address unit's queue is full 14%; waves wait for data or the barrier 32% and to issue 37%
 // of theirs, with two of them per SIMD to cover it. (Two sets of waves in opposite phases, one forming S while the other ran
